@@ -209,7 +209,9 @@ int sph_set_rebuild_kernel(sph_ctx *ctx, int fused);
  * that runs past it ends the kernel on every block, the list and contact
  * kernels after it skip their work, and the step returns SPH_ERR_HIP; a
  * small bound forces that path from the host, for tests of the failure
- * handling.  Takes effect at once. */
+ * handling.  It also bounds the polls of a fluid's resident iterations
+ * (default 2^20); where one runs out the solve is repeated with one launch
+ * per sweep, as are the later ones.  Takes effect at once. */
 int sph_set_barrier_spin_limit(sph_ctx *ctx, uint32_t sleeps);
 
 /* Load a state: replaces DEM::readbin + checkValues + transfer to the device

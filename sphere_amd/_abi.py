@@ -394,7 +394,8 @@ class Engine:
         return s
 
     def set_barrier_spin_limit(self, sleeps):
-        """Bound of the list rebuild kernel's grid-barrier waits (0: default)."""
+        """Bound of the list rebuild kernel's grid-barrier waits and of the
+        fluid's resident iterations (0: defaults)."""
         self._check(self.lib.sph_set_barrier_spin_limit(self.ctx, int(sleeps)))
 
     def set_profiling(self, on):

@@ -735,6 +735,34 @@ __device__ __forceinline__ double jacobi_target(const DarcyArgs &d, const double
     return jc[j.base + i] + epsilon * dp_impl;
 }
 
+// the ghost cells of a scalar field that copy interior cell (x, y, z)
+// (k_ghosts' rules), whose value is v
+__device__ __forceinline__ void copy_ghosts(const DarcyArgs &d, int x, int y, int z, double v,
+                                            double *__restrict__ p)
+{
+    const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
+#define GW(X, Y, Z) p[didx(d, X, Y, Z)] = v
+    if (x == 0 && d.bc_xn == 0) GW(-1, y, z);
+    if (x == 1 && d.bc_xn == 1) GW(-1, y, z);
+    if (x == 0 && d.bc_xn == 2) GW(nx, y, z);
+    if (x == nx - 1 && d.bc_xp == 0) GW(nx, y, z);
+    if (x == nx - 2 && d.bc_xp == 1) GW(nx, y, z);
+    if (x == nx - 1 && d.bc_xp == 2) GW(-1, y, z);
+    if (y == 0 && d.bc_yn == 0) GW(x, -1, z);
+    if (y == 1 && d.bc_yn == 1) GW(x, -1, z);
+    if (y == 0 && d.bc_yn == 2) GW(x, ny, z);
+    if (y == ny - 1 && d.bc_yp == 0) GW(x, ny, z);
+    if (y == ny - 2 && d.bc_yp == 1) GW(x, ny, z);
+    if (y == ny - 1 && d.bc_yp == 2) GW(x, -1, z);
+    if (z == 0 && d.bc_bot == 0) GW(x, y, -1);
+    if (z == 1 && d.bc_bot == 1) GW(x, y, -1);
+    if (z == 0 && d.bc_bot == 2) GW(x, y, nz);
+    if (z == nz - 1 && d.bc_top == 0) GW(x, y, nz);
+    if (z == nz - 2 && d.bc_top == 1) GW(x, y, nz);
+    if (z == nz - 1 && d.bc_top == 2) GW(x, y, -1);
+#undef GW
+}
+
 // One sweep of the Jacobi loop body (src/device.cu:2184-2331) in a single
 // launch: updateDarcySolution on iterate p_in into p_out, then, into p_out,
 // the ghost values that the next sweep's setDarcyGhostNodes would copy from
@@ -778,7 +806,7 @@ __device__ __forceinline__ void darcy_sweep_body(DarcyArgs d, const double *__re
     unsigned long long bits = 0;
     if (clear && i < RED_LANES) clear[i * RED_STRIDE] = 0ull;
     if (i < n) {
-        const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
+        const int nz = (int)d.nz;
         const int x = (int)(i % d.nx), y = (int)((i / d.nx) % d.ny), z = (int)(i / (d.nx * d.ny));
         const uint32_t c = didx(d, x, y, z);
         const double p = p_in[c];
@@ -787,26 +815,7 @@ __device__ __forceinline__ void darcy_sweep_body(DarcyArgs d, const double *__re
         p_new = p * (1.0 - theta) + p_new * theta;
         const double res_norm = (p_new - p) / (p + 1.0e-16);
         p_out[c] = p_new;
-#define GW(X, Y, Z) p_out[didx(d, X, Y, Z)] = p_new
-        if (x == 0 && d.bc_xn == 0) GW(-1, y, z);
-        if (x == 1 && d.bc_xn == 1) GW(-1, y, z);
-        if (x == 0 && d.bc_xn == 2) GW(nx, y, z);
-        if (x == nx - 1 && d.bc_xp == 0) GW(nx, y, z);
-        if (x == nx - 2 && d.bc_xp == 1) GW(nx, y, z);
-        if (x == nx - 1 && d.bc_xp == 2) GW(-1, y, z);
-        if (y == 0 && d.bc_yn == 0) GW(x, -1, z);
-        if (y == 1 && d.bc_yn == 1) GW(x, -1, z);
-        if (y == 0 && d.bc_yn == 2) GW(x, ny, z);
-        if (y == ny - 1 && d.bc_yp == 0) GW(x, ny, z);
-        if (y == ny - 2 && d.bc_yp == 1) GW(x, ny, z);
-        if (y == ny - 1 && d.bc_yp == 2) GW(x, -1, z);
-        if (z == 0 && d.bc_bot == 0) GW(x, y, -1);
-        if (z == 1 && d.bc_bot == 1) GW(x, y, -1);
-        if (z == 0 && d.bc_bot == 2) GW(x, y, nz);
-        if (z == nz - 1 && d.bc_top == 0) GW(x, y, nz);
-        if (z == nz - 2 && d.bc_top == 1) GW(x, y, nz);
-        if (z == nz - 1 && d.bc_top == 2) GW(x, y, -1);
-#undef GW
+        copy_ghosts(d, x, y, z, p_new, p_out);
         if ((z == 0 && d.bc_bot == 4) || (z == nz - 1 && d.bc_top == 4)) {
             const double q_z = z == 0 ? d.bc_bot_flux : d.bc_top_flux;
             const double p_ghost = -d.mu / k_a[c] * q_z * (d.L2 / nz) + p;
@@ -860,6 +869,125 @@ void launch_darcy_sweep(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b
                        b.k, p_out, check, clear, prev, tolerance, prev_nijac,
                        b.maxres + (free_running ? DARCY_ZERO : DARCY_STATE),
                        zero_scale ? b.maxres + DARCY_SCALE : (unsigned long long *)nullptr);
+}
+
+// A cell of the sweep in a resident launch (resident.h): the solve's
+// constants in registers, the same expressions as jacobi_target and
+// darcy_sweep_body.  Flux boundaries (their ghosts lag a sweep) and axes
+// periodic on one side only are left to the launch per sweep
+// (darcy_resident_form).
+struct DarcyOp {
+    typedef unsigned long long State;
+    DarcyArgs d;
+    const double *jc;
+    const uint8_t *frozen;
+    const double *p_in;
+    double *p_out;
+    unsigned long long *st;
+    unsigned long long *scale;  // cleared for the correction that may follow
+    double tolerance;
+    FixedDiv hx, hy, hz;  // the cell's edges
+    struct Cell {
+        double h[6], A, F, base;
+        unsigned bits;  // bit k: the neighbour in direction k is a ghost with this cell's value; 6: frozen
+    };
+    __device__ State *state() const { return st; }
+    __device__ double in(int x, int y, int z) const { return p_in[didx(d, x, y, z)]; }
+    __device__ void load(Cell &c, int x, int y, int z) const
+    {
+        const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
+        const JLayout j = jlayout(d);
+        const size_t i = (size_t)x + d.nx * ((size_t)y + d.ny * (size_t)z);
+        const size_t fx = (size_t)x + j.sxf * ((size_t)y + d.ny * (size_t)z);
+        const size_t fy = j.hy + (size_t)x + d.nx * ((size_t)y + j.syf * (size_t)z);
+        c.h[0] = jc[fx];
+        c.h[1] = jc[fx + 1];
+        c.h[2] = jc[fy];
+        c.h[3] = jc[fy + d.nx];
+        c.h[4] = jc[j.hz + i];
+        c.h[5] = jc[j.hz + i + (size_t)d.nx * d.ny];
+        c.A = jc[j.A + i];
+        c.F = jc[j.F + i];
+        c.base = jc[j.base + i];
+        c.bits = (x == 0 && d.bc_xn != 2 ? 1u : 0u) | (x == nx - 1 && d.bc_xp != 2 ? 2u : 0u) |
+                 (y == 0 && d.bc_yn != 2 ? 4u : 0u) | (y == ny - 1 && d.bc_yp != 2 ? 8u : 0u) |
+                 (z == 0 && d.bc_bot != 2 ? 16u : 0u) | (z == nz - 1 && d.bc_top != 2 ? 32u : 0u) |
+                 (frozen[i] ? 64u : 0u);
+    }
+    template <bool FIXED>
+    __device__ double next(const Cell &c, double p, double p_xn, double p_xp, double p_yn, double p_yp,
+                           double p_zn, double p_zp) const
+    {
+#define D(N, H) div_by<FIXED>(N, H)
+        const double div_k_grad_p = D(D(c.h[1] * (p_xp - p), hx) - D(c.h[0] * (p - p_xn), hx), hx) +
+                                    D(D(c.h[3] * (p_yp - p), hy) - D(c.h[2] * (p - p_yn), hy), hy) +
+                                    D(D(c.h[5] * (p_zp - p), hz) - D(c.h[4] * (p - p_zn), hz), hz);
+#undef D
+        double dp_impl = c.A * div_k_grad_p - c.F;
+        if (c.bits & 64u) dp_impl = 0.0;
+        const double epsilon = 0.5;
+        const double target = c.base + epsilon * dp_impl;
+        const double theta = 0.05;
+        return p * (1.0 - theta) + target * theta;
+    }
+    __device__ double step(Cell &c, double p, double p_xn, double p_xp, double p_yn, double p_yp, double p_zn,
+                           double p_zp, bool check, unsigned long long &bits) const
+    {
+        const unsigned b = c.bits;
+        if (b & 1u) p_xn = p;
+        if (b & 2u) p_xp = p;
+        if (b & 4u) p_yn = p;
+        if (b & 8u) p_yp = p;
+        if (b & 16u) p_zn = p;
+        if (b & 32u) p_zp = p;
+        double p_new = next<true>(c, p, p_xn, p_xp, p_yn, p_yp, p_zn, p_zp);
+        if (!(fabs(p_new) < 1.0e300)) p_new = next<false>(c, p, p_xn, p_xp, p_yn, p_yp, p_zn, p_zp);
+        if (check) bits = (unsigned long long)__double_as_longlong(fabs((p_new - p) / (p + 1.0e-16)));
+        return p_new;
+    }
+    __device__ unsigned verdict(unsigned long long m, unsigned) const
+    {
+        const double v = __longlong_as_double((long long)m);
+        return v != v ? 2u : v <= tolerance ? 1u : 0u;
+    }
+    __device__ void record(unsigned long long m, unsigned it, unsigned verdict) const
+    {
+        st[1] = it;
+        st[2] = m;
+        if (verdict) atomicMax(st, (unsigned long long)verdict);
+    }
+    __device__ void finish(int x, int y, int z, double value, double) const
+    {
+        p_out[didx(d, x, y, z)] = value;
+        copy_ghosts(d, x, y, z, value, p_out);
+        const uint32_t n = d.nx * d.ny * d.nz;
+        for (uint32_t i = (uint32_t)x + d.nx * ((uint32_t)y + d.ny * (uint32_t)z); i < RED_LANES; i += n)
+            scale[i * RED_STRIDE] = 0ull;
+    }
+};
+
+// What a resident launch computes as the sweeps do: on each axis both
+// boundaries periodic, or neither and each either fixed (0) or mirrored (1).
+bool darcy_resident_form(const DarcyArgs &d, int &wrap)
+{
+    const int b[3][2] = {{d.bc_xn, d.bc_xp}, {d.bc_yn, d.bc_yp}, {d.bc_bot, d.bc_top}};
+    wrap = 0;
+    for (int k = 0; k < 3; ++k) {
+        if (b[k][0] == 2 && b[k][1] == 2) wrap |= 1 << k;
+        else if (b[k][0] < 0 || b[k][0] > 1 || b[k][1] < 0 || b[k][1] > 1) return false;
+    }
+    return true;
+}
+
+// Sweeps [a.it0, a.it1) from p_in into p_out (ghosts included); a.it0's
+// verdicts go into the solve state like those of the single sweeps.
+void launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
+                           const DarcyArgs &d, const DarcyBuffers &b, const double *p_in, double *p_out,
+                           double tolerance)
+{
+    const DarcyOp op{d, b.jc, b.jfrozen, p_in, p_out, b.maxres + DARCY_STATE, b.maxres + DARCY_SCALE, tolerance,
+                     fixed_div(d.dx), fixed_div(d.dy), fixed_div(d.dz)};
+    resident_launch(r, device, s, a, op);
 }
 
 // The test of a check sweep that no sweep follows (the last of maxiter).
@@ -1005,30 +1133,8 @@ __device__ __forceinline__ void darcy_net_apply_body(DarcyArgs d, const uint8_t 
     const int x = (int)(i % d.nx), y = (int)((i / d.nx) % d.ny), z = (int)(i / (d.nx * d.ny));
     double &pc = p[didx(d, x, y, z)];
     pc += s * (double)ev;
-    // the ghost cells that copy this cell (k_ghosts' rules for a scalar
-    // field); the other ghosts already hold the unchanged cells' values
-    const double v = pc;
-    const int nx = (int)d.nx, ny = (int)d.ny, nz = (int)d.nz;
-#define GW(X, Y, Z) p[didx(d, X, Y, Z)] = v
-    if (x == 0 && d.bc_xn == 0) GW(-1, y, z);
-    if (x == 1 && d.bc_xn == 1) GW(-1, y, z);
-    if (x == 0 && d.bc_xn == 2) GW(nx, y, z);
-    if (x == nx - 1 && d.bc_xp == 0) GW(nx, y, z);
-    if (x == nx - 2 && d.bc_xp == 1) GW(nx, y, z);
-    if (x == nx - 1 && d.bc_xp == 2) GW(-1, y, z);
-    if (y == 0 && d.bc_yn == 0) GW(x, -1, z);
-    if (y == 1 && d.bc_yn == 1) GW(x, -1, z);
-    if (y == 0 && d.bc_yn == 2) GW(x, ny, z);
-    if (y == ny - 1 && d.bc_yp == 0) GW(x, ny, z);
-    if (y == ny - 2 && d.bc_yp == 1) GW(x, ny, z);
-    if (y == ny - 1 && d.bc_yp == 2) GW(x, -1, z);
-    if (z == 0 && d.bc_bot == 0) GW(x, y, -1);
-    if (z == 1 && d.bc_bot == 1) GW(x, y, -1);
-    if (z == 0 && d.bc_bot == 2) GW(x, y, nz);
-    if (z == nz - 1 && d.bc_top == 0) GW(x, y, nz);
-    if (z == nz - 2 && d.bc_top == 1) GW(x, y, nz);
-    if (z == nz - 1 && d.bc_top == 2) GW(x, y, -1);
-#undef GW
+    // the other ghosts already hold the unchanged cells' values
+    copy_ghosts(d, x, y, z, pc, p);
 }
 
 __global__ void __launch_bounds__(256) k_darcy_net_apply(DarcyArgs d, const uint8_t *__restrict__ frozen,

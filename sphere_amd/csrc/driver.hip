@@ -85,6 +85,7 @@ struct sph_ctx {
     unsigned long long *h_u64 = nullptr;
     unsigned long long *h_state = nullptr;  // Jacobi solve state (4 words)
     unsigned int jacobi_hint = 0;           // sweeps of the last solve
+    Resident res;                           // tiles and inboxes of the resident sweeps
     double *h_d = nullptr;
     // learned Darcy correction: host parameters, and the network with its
     // device buffers for the loaded grid (made at the first solve)
@@ -249,6 +250,7 @@ static void free_device(sph_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->aux) (void)hipStreamSynchronize(ctx->aux);
     ctx->walls_pending = false;
+    resident_free(ctx->res);
     for (void *p : ctx->allocs) (void)hipFree(p);
     ctx->allocs.clear();
     ctx->db = DemBuffers{};
@@ -781,6 +783,77 @@ static int net_ready(sph_ctx *ctx)
     return sync(ctx);
 }
 
+// The learned correction of iterate pc; its kernels do nothing once the solve
+// has ended.  The input goes straight into the network's BF16 rows, and the
+// correction refreshes the ghosts of the cells it changes.
+static int darcy_correct(sph_ctx *ctx, const DarcyArgs &da, double *pc)
+{
+    hipStream_t s = ctx->stream;
+    const DarcyBuffers &d = ctx->dd;
+    launch_darcy_residual_max(s, da, d, pc, false);
+    launch_darcy_net_input(s, da, d, pc, nullptr, false, net_input_bf16(ctx->net));
+    const int rc = net_forward_packed(ctx->net, ctx->net_params, nullptr, ctx->net_out, s);
+    if (rc) return fail(ctx, rc, sph_net_last_error());
+    launch_darcy_net_apply(s, da, d, pc, ctx->net_out);
+    return SPH_OK;
+}
+
+// The sweeps of a solve as resident launches (resident.h): one launch up to
+// each learned correction (after sweeps 1, 11, 21, ...), then one to the end.
+// The launches alternate between the two iterate buffers; out is the one that
+// holds the solve's result, h_state the solve state.  With resident = false
+// on return a wait ran out: the solve is back at its start, and this context
+// goes on with one launch per sweep.
+static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2], bool &resident, int &out)
+{
+    const sph_state &h = ctx->hs.h;
+    hipStream_t s = ctx->stream;
+    const DarcyBuffers &d = ctx->dd;
+    const unsigned int chunk = 20000u;  // sweeps of a launch: some 30 ms
+    std::vector<unsigned int> ends;
+    int corrections = 0, cur = 0;
+    std::memset(ctx->h_state, 0, 32);
+    for (unsigned int it = 0; it < h.maxiter && ctx->h_state[0] == 0;) {
+        const bool learned = ctx->net && corrections < ctx->net_max_corr;
+        const unsigned int len = learned ? (it == 0 ? 2u : 10u) : chunk;
+        const unsigned int end = it + std::min(len, h.maxiter - it);
+        ResidentArgs a;
+        bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->rb_spin, a);
+        if (ok) {
+            ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
+            launch_darcy_resident(s, ctx->device, ctx->res, a, da, d, buf[cur], buf[cur ^ 1], h.tolerance);
+            cur ^= 1;
+            ends.push_back(end);
+            if (learned && end % 10u == 2u) {
+                const int rc = darcy_correct(ctx, da, buf[cur]);
+                if (rc) return rc;
+                ++corrections;
+            }
+        }
+        it = end;
+        // wait for the state where the last solve ended, and after the
+        // launches that run to the end
+        if (ok && learned && it < h.maxiter && it < ctx->jacobi_hint) continue;
+        HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
+        const int rc = sync(ctx);
+        if (rc) return rc;
+        if (!ok || ctx->h_state[0] == RES_ABORT) {
+            ctx->res.usable = false;
+            resident = false;
+            launch_darcy_copy_interior(s, da, d.p_old, buf[0]);
+            launch_darcy_ghosts(s, da, buf[0], 1);
+            launch_fill_u32(s, (uint32_t *)d.maxres, 2 * DARCY_MAXRES_WORDS, 0u);
+            return SPH_OK;
+        }
+    }
+    // launch k writes buffer (k + 1) & 1
+    size_t k = ends.empty() ? 0 : ends.size() - 1;
+    if (ctx->h_state[0] != 0)
+        for (k = 0; ends[k] <= ctx->h_state[1];) ++k;
+    out = ends.empty() ? 0 : (int)((k + 1) & 1u);
+    return SPH_OK;
+}
+
 // Darcy branch of the loop body, src/device.cu:1901-2426
 static int darcy_step(sph_ctx *ctx, std::ofstream *convlog)
 {
@@ -837,58 +910,70 @@ static int darcy_step(sph_ctx *ctx, std::ofstream *convlog)
     double *buf[2] = {d.p, d.p_new};
     int rc0 = net_ready(ctx);
     if (rc0) return rc0;
-    int corrections = 0;
-    unsigned int nijac = 0;
     unsigned long long state = 0, last_nijac = 0, last_bits = 0;
-    unsigned long long want = std::max(12u, (ctx->jacobi_hint + 9u) / 10u * 10u + 2u);
-    while (nijac < h.maxiter && state == 0) {
-        const unsigned int end = (unsigned int)std::min<unsigned long long>(h.maxiter, want);
-        for (; nijac < end; ++nijac) {
-            const bool check = (nijac % 10 == 0);
-            // two check slots alternate: a check sweep zeroes the other one
-            unsigned long long *slot = d.maxres + ((nijac / 10) & 1u) * RED_WORDS;
-            unsigned long long *next = d.maxres + (((nijac / 10) & 1u) ^ 1u) * RED_WORDS;
-            const bool decides = nijac > 0 && (nijac - 1) % 10 == 0;
-            const unsigned long long *prev = decides ? d.maxres + (((nijac - 1) / 10) & 1u) * RED_WORDS : nullptr;
-            ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
-            // setDarcyTopWallFixedFlow (bc_top == 1) writes dev_darcy_p, which
-            // the copy of p_new into p overwrites: it has no effect
-            // (device.cu:2284-2331)
-            // learned correction of the iterate this deciding sweep wrote
-            // (its kernels do nothing once the solve has ended); the sweep
-            // clears the correction's scale slot
-            const bool correct = decides && ctx->net && corrections < ctx->net_max_corr;
-            launch_darcy_sweep(s, da, d, buf[nijac & 1u], buf[(nijac & 1u) ^ 1u],
-                               check ? slot : nullptr, check ? next : nullptr, prev, h.tolerance,
-                               nijac - 1u, false, correct);
-            if (correct) {
-                double *pc = buf[(nijac & 1u) ^ 1u];
-                launch_darcy_residual_max(s, da, d, pc, false);
-                // the input goes straight into the network's BF16 rows, and
-                // the correction refreshes the ghosts of the cells it changes
-                launch_darcy_net_input(s, da, d, pc, nullptr, false, net_input_bf16(ctx->net));
-                int nrc = net_forward_packed(ctx->net, ctx->net_params, nullptr, ctx->net_out, s);
-                if (nrc) return fail(ctx, nrc, sph_net_last_error());
-                launch_darcy_net_apply(s, da, d, pc, ctx->net_out);
-                ++corrections;
-            }
+    int out = 0;  // the buffer holding the solve's result
+    int wrap = 0;
+    bool resident = darcy_resident_form(da, wrap);
+    if (resident && !ctx->res.planned)
+        resident_plan(ctx->res, ctx->device, (int)da.nx, (int)da.ny, (int)da.nz, wrap);
+    resident = resident && ctx->res.usable;
+    if (resident) {
+        rc0 = darcy_resident(ctx, da, buf, resident, out);
+        if (rc0) return rc0;
+        if (resident) {
+            state = ctx->h_state[0];
+            last_nijac = ctx->h_state[1];
+            last_bits = ctx->h_state[2];
         }
-        if (nijac == h.maxiter && (h.maxiter - 1) % 10 == 0)
-            launch_darcy_decide(s, d, d.maxres + (((h.maxiter - 1) / 10) & 1u) * RED_WORDS, h.tolerance,
-                                h.maxiter - 1);
-        HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
-        int rc = sync(ctx);
-        if (rc) return rc;
-        state = ctx->h_state[0];
-        last_nijac = ctx->h_state[1];
-        last_bits = ctx->h_state[2];
-        want = (unsigned long long)nijac + 20u;
+    }
+    if (!resident) {
+        int corrections = 0;
+        unsigned int nijac = 0;
+        unsigned long long want = std::max(12u, (ctx->jacobi_hint + 9u) / 10u * 10u + 2u);
+        while (nijac < h.maxiter && state == 0) {
+            const unsigned int end = (unsigned int)std::min<unsigned long long>(h.maxiter, want);
+            for (; nijac < end; ++nijac) {
+                const bool check = (nijac % 10 == 0);
+                // two check slots alternate: a check sweep zeroes the other one
+                unsigned long long *slot = d.maxres + ((nijac / 10) & 1u) * RED_WORDS;
+                unsigned long long *next = d.maxres + (((nijac / 10) & 1u) ^ 1u) * RED_WORDS;
+                const bool decides = nijac > 0 && (nijac - 1) % 10 == 0;
+                const unsigned long long *prev = decides ? d.maxres + (((nijac - 1) / 10) & 1u) * RED_WORDS : nullptr;
+                ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
+                // setDarcyTopWallFixedFlow (bc_top == 1) writes dev_darcy_p, which
+                // the copy of p_new into p overwrites: it has no effect
+                // (device.cu:2284-2331)
+                // learned correction of the iterate this deciding sweep wrote
+                // (its kernels do nothing once the solve has ended); the sweep
+                // clears the correction's scale slot
+                const bool correct = decides && ctx->net && corrections < ctx->net_max_corr;
+                launch_darcy_sweep(s, da, d, buf[nijac & 1u], buf[(nijac & 1u) ^ 1u],
+                                   check ? slot : nullptr, check ? next : nullptr, prev, h.tolerance,
+                                   nijac - 1u, false, correct);
+                if (correct) {
+                    const int nrc = darcy_correct(ctx, da, buf[(nijac & 1u) ^ 1u]);
+                    if (nrc) return nrc;
+                    ++corrections;
+                }
+            }
+            if (nijac == h.maxiter && (h.maxiter - 1) % 10 == 0)
+                launch_darcy_decide(s, d, d.maxres + (((h.maxiter - 1) / 10) & 1u) * RED_WORDS, h.tolerance,
+                                    h.maxiter - 1);
+            HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
+            int rc = sync(ctx);
+            if (rc) return rc;
+            state = ctx->h_state[0];
+            last_nijac = ctx->h_state[1];
+            last_bits = ctx->h_state[2];
+            want = (unsigned long long)nijac + 20u;
+        }
     }
     ctx->stats.corrections += ctx->h_state[3];
     // sweeps that ran: up to the deciding check, or all maxiter
     const unsigned int ran = state != 0 ? (unsigned int)last_nijac + 1u : h.maxiter;
-    d.p = buf[ran & 1u];
-    d.p_new = buf[(ran & 1u) ^ 1u];
+    if (!resident) out = (int)(ran & 1u);
+    d.p = buf[out];
+    d.p_new = buf[out ^ 1];
     ctx->stats.sweeps += ran;
     ctx->jacobi_hint = ran;
     double max_norm_res;
@@ -1247,7 +1332,8 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
         rc = ns_coupled_step(ctx->ns, h.np, (const double *)ctx->db.x, (const double *)ctx->db.vel,
                              (const double *)ctx->db.x_s, ctx->db.cell_start, ctx->db.cell_end, ctx->db.vals,
                              h.origo, h.periodic, (double *)ctx->db.force,
-                             h.nw > 0 && (h.wmode[0] == 1 || h.wmode[0] == 3) ? ctx->host_wx0 : -1.0, s);
+                             h.nw > 0 && (h.wmode[0] == 1 || h.wmode[0] == 3) ? ctx->host_wx0 : -1.0,
+                             ctx->rb_spin, s);
         if (rc) return fail(ctx, rc, sph_ns_last_error());
     }
     if (h.np > 0) {
@@ -1974,6 +2060,7 @@ struct sph_ensemble {
     std::vector<uint64_t> fl_gen;
     std::vector<uint32_t> fl_parity;
     std::vector<uint32_t *> fl_keys;
+    std::vector<double *> fl_p;  // the buffer every box's pressure is in
     bool fl_planned = false;
     uint32_t fl_phase = 0;
     EnsFluidPhase fph[2];
@@ -2452,6 +2539,7 @@ static int ens_fluid_plan(sph_ensemble *e)
     e->fl_gen.clear();
     e->fl_parity.clear();
     e->fl_keys.clear();
+    e->fl_p.clear();
     if (e->fluid.empty()) {
         e->fl_planned = true;
         return SPH_OK;
@@ -2466,6 +2554,7 @@ static int ens_fluid_plan(sph_ensemble *e)
         e->fl_gen.push_back(c->gen);
         e->fl_parity.push_back(c->nl_parity);
         e->fl_keys.push_back(c->db.keys);
+        e->fl_p.push_back(c->dd.p);
     }
     e->fl_maxiter = e->boxes[e->fluid[0]]->hs.h.maxiter;
     e->fl_phase = 0;
@@ -2620,7 +2709,7 @@ static bool ens_fluid_current(const sph_ensemble *e)
         if (ens_fluid_eligible(c) != (e->fl_elig[k] != 0)) return false;
         const bool in = i < e->fluid.size() && e->fluid[i] == (int)k;
         if (!in) continue;
-        if (c->gen != e->fl_gen[i]) return false;
+        if (c->gen != e->fl_gen[i] || c->dd.p != e->fl_p[i]) return false;
         if (c->nl_parity != (e->fl_parity[i] ^ e->fl_phase)) return false;
         const bool swapped = (radix_passes(c) & 1) != 0 && e->fl_phase == 1;
         if ((c->db.keys == e->fl_keys[i]) == swapped) return false;

@@ -5,6 +5,7 @@
 
 #include "common.h"
 #include "multi.h"
+#include "resident.h"
 
 // Step counter and simulation time on the device (read by integrate and the
 // wall integration, advanced by k_clock_advance after them), so that a step
@@ -342,6 +343,11 @@ void launch_darcy_sweep(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b
                         unsigned long long *clear, const unsigned long long *prev,
                         double tolerance, uint32_t prev_nijac, bool free_running = false,
                         bool zero_scale = false);
+// sweeps in one resident launch (resident.h), where the boundaries allow it
+bool darcy_resident_form(const DarcyArgs &d, int &wrap);
+void launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
+                           const DarcyArgs &d, const DarcyBuffers &b, const double *p_in, double *p_out,
+                           double tolerance);
 void launch_darcy_residual_max(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b, const double *p,
                                bool free_running);
 // the network input of iterate p: FP32 rows of 3 (input) and/or the

@@ -36,6 +36,7 @@
 #include "../../include/sphere_hip.h"
 #include "multi.h"
 #include "ns.h"
+#include "resident.h"
 
 namespace {
 
@@ -522,6 +523,30 @@ struct NsSolveState {
     unsigned long long maxw, lastmax;
 };
 
+// The parts of the forcing that do not change within a solve (findNSforcing,
+// src/navierstokes.cuh:2497-2617): f1 and grad phi / phi of a cell.
+__device__ inline void forcing_terms(const NsGrid &g, const NsPhys &q, const CVec3 &VPc, const CVec3 &VPF,
+                                     const double *phi_a, const double *dphi_a, int x, int y, int z,
+                                     double &f1, double f2[3])
+{
+    const double dx = g.dx, dy = g.dy, dz = g.dz;
+    const size_t c = cidx(g, x, y, z);
+    const double phi = phi_a[c], dphi = dphi_a[c];
+    const double div_v_p = (VPF.c[0][fidx(g, x + 1, y, z)] - VPF.c[0][fidx(g, x, y, z)]) / dx +
+                           (VPF.c[1][fidx(g, x, y + 1, z)] - VPF.c[1][fidx(g, x, y, z)]) / dy +
+                           (VPF.c[2][fidx(g, x, y, z + 1)] - VPF.c[2][fidx(g, x, y, z)]) / dz;
+    const double gp[3] = {(phi_a[cidx(g, x + 1, y, z)] - phi_a[cidx(g, x - 1, y, z)]) / (2.0 * dx),
+                          (phi_a[cidx(g, x, y + 1, z)] - phi_a[cidx(g, x, y - 1, z)]) / (2.0 * dy),
+                          (phi_a[cidx(g, x, y, z + 1)] - phi_a[cidx(g, x, y, z - 1)]) / (2.0 * dz)};
+    const double dt = q.dt;
+    const double dot_gv = gp[0] * VPc.c[0][c] + gp[1] * VPc.c[1][c] + gp[2] * VPc.c[2][c];
+    const double t1 = q.rho_f * div_v_p / (q.c_v * dt);
+    const double t2 = q.rho_f * dot_gv / (q.c_v * dt * phi);
+    const double t4 = q.rho_f * dphi / (dt * dt * phi * q.c_v);
+    f1 = t1 + t2 + t4;
+    for (int k = 0; k < 3; ++k) f2[k] = gp[k] / phi;
+}
+
 // One Jacobi iteration: findNSforcing (src/navierstokes.cuh:2497-2617),
 // setNSghostNodes(epsilon), jacobiIterationNS (:2679-2792, no wall) and
 // copyValues (:2795-2827), A -> B, as described at the top of this file.
@@ -539,20 +564,7 @@ k_ns_jacobi(NsGrid g, NsPhys q, unsigned nijac, const double *A, double *B, doub
         const size_t c = cidx(g, x, y, z);
         double f1, f2[3];
         if (nijac == 0) {
-            const double phi = phi_a[c], dphi = dphi_a[c];
-            const double div_v_p = (VPF.c[0][fidx(g, x + 1, y, z)] - VPF.c[0][fidx(g, x, y, z)]) / dx +
-                                   (VPF.c[1][fidx(g, x, y + 1, z)] - VPF.c[1][fidx(g, x, y, z)]) / dy +
-                                   (VPF.c[2][fidx(g, x, y, z + 1)] - VPF.c[2][fidx(g, x, y, z)]) / dz;
-            const double gp[3] = {(phi_a[cidx(g, x + 1, y, z)] - phi_a[cidx(g, x - 1, y, z)]) / (2.0 * dx),
-                                  (phi_a[cidx(g, x, y + 1, z)] - phi_a[cidx(g, x, y - 1, z)]) / (2.0 * dy),
-                                  (phi_a[cidx(g, x, y, z + 1)] - phi_a[cidx(g, x, y, z - 1)]) / (2.0 * dz)};
-            const double dt = q.dt;
-            const double dot_gv = gp[0] * VPc.c[0][c] + gp[1] * VPc.c[1][c] + gp[2] * VPc.c[2][c];
-            const double t1 = q.rho_f * div_v_p / (q.c_v * dt);
-            const double t2 = q.rho_f * dot_gv / (q.c_v * dt * phi);
-            const double t4 = q.rho_f * dphi / (dt * dt * phi * q.c_v);
-            f1 = t1 + t2 + t4;
-            for (int k = 0; k < 3; ++k) f2[k] = gp[k] / phi;
+            forcing_terms(g, q, VPc, VPF, phi_a, dphi_a, x, y, z, f1, f2);
             f1a[c] = f1;
             for (int k = 0; k < 3; ++k) f2a.c[k][c] = f2[k];
         } else {
@@ -616,6 +628,120 @@ __global__ void k_ns_decide(NsSolveState *st, unsigned nijac, double tolerance)
         st->conv_nijac = nijac;
     }
 }
+
+// The same iteration for a cell of a resident launch (resident.h), from its
+// value e and its neighbours' in the current iterate.  Two kinds of ghost
+// neighbour occur, as above: the stencil takes the interior cell that the
+// ghost rules copy, the forcing takes the ghost layer, which holds that
+// cell's value of the iteration before (the array's ghost layer at first).
+// lag[k] is the lagging neighbour on axis k of a cell at that axis' end.
+struct NsOp {
+    typedef unsigned State;
+    NsGrid g;
+    NsPhys q;
+    const double *A;
+    double *B;
+    CVec3 VPc, VPF;
+    const double *phi, *dphi;
+    NsSolveState *st;
+    double tolerance, dp_dz;
+    unsigned wall0_iz;
+    FixedDiv h2x, h2y, h2z, denom;  // 2 dx, 2 dy, 2 dz; the stencil's denominator
+    struct Cell {
+        double f1, f2[3], lag[3];
+        unsigned bits;  // ends: bit 2 k low, bit 2 k + 1 high end of axis k; then the cases below
+    };
+    static constexpr unsigned FREE = 64u, WALL = 128u, ABOVE = 256u, ZP_IS_ZN = 512u, ZN_OWN = 1024u,
+                              ZP_OWN = 2048u, GRAD = 4096u;
+    __device__ State *state() const { return &st->done; }
+    __device__ double in(int x, int y, int z) const { return A[cidx(g, x, y, z)]; }
+    __device__ void load(Cell &c, int x, int y, int z) const
+    {
+        forcing_terms(g, q, VPc, VPF, phi, dphi, x, y, z, c.f1, c.f2);
+        const int X[3] = {x, y, z}, n[3] = {g.nx, g.ny, g.nz};
+        unsigned b = 0u;
+        for (int k = 0; k < 3; ++k) {
+            int lo[3] = {x, y, z}, hi[3] = {x, y, z};
+            lo[k] = -1;
+            hi[k] = n[k];
+            c.lag[k] = 0.0;
+            if (X[k] == 0) {
+                b |= 1u << (2 * k);
+                c.lag[k] = A[cidx(g, lo[0], lo[1], lo[2])];
+            }
+            if (X[k] == n[k] - 1) {
+                b |= 2u << (2 * k);
+                c.lag[k] = A[cidx(g, hi[0], hi[1], hi[2])];
+            }
+        }
+        const int zmin = g.bb == 0 ? 1 : 0;
+        const int zmax = g.bt == 0 ? g.nz - 2 : g.nz - 1;
+        if (z >= zmin && z <= zmax) b |= FREE;
+        if ((unsigned)z == wall0_iz) b |= WALL;
+        if ((unsigned)z == wall0_iz + 1u) b |= ABOVE;
+        if (z == 0 && g.bb != 2) b |= ZN_OWN;
+        if (z == g.nz - 1 && g.bt == 0) b |= ZP_OWN;
+        if (z == g.nz - 1 && g.bt == 1) b |= ZP_IS_ZN;
+        if (c.f2[0] != 0.0 || c.f2[1] != 0.0 || c.f2[2] != 0.0) b |= GRAD;
+        c.bits = b;
+    }
+    // dx_, dy_, dz_: the forcing's differences; ex, ey, ez: the stencil's sums
+    template <bool FIXED>
+    __device__ double next(const Cell &c, double dx_, double dy_, double dz_, double ex, double ey,
+                           double ez) const
+    {
+        double f = c.f1;
+        // where the porosity is uniform grad eps is multiplied by zeros
+        if (!FIXED || (c.bits & GRAD))
+            f = c.f1 - (div_by<FIXED>(dx_, h2x) * c.f2[0] + div_by<FIXED>(dy_, h2y) * c.f2[1] +
+                        div_by<FIXED>(dz_, h2z) * c.f2[2]);
+        const double dxdx = g.dx * g.dx, dydy = g.dy * g.dy, dzdz = g.dz * g.dz;
+        return div_by<FIXED>(-dxdx * dydy * dzdz * f + dydy * dzdz * ex + dxdx * dzdz * ey + dxdx * dydy * ez,
+                             denom);
+    }
+    __device__ double step(Cell &c, double e, double e_xn, double e_xp, double e_yn, double e_yp, double e_zn,
+                           double e_zp, bool check, unsigned long long &bits) const
+    {
+        const unsigned b = c.bits;
+        if (b & ZN_OWN) e_zn = e;
+        if (b & ZP_OWN) e_zp = e;
+        if (b & ZP_IS_ZN) e_zp = e_zn;
+        const double dx_ = ((b & 2u) ? c.lag[0] : e_xp) - ((b & 1u) ? c.lag[0] : e_xn);
+        const double dy_ = ((b & 8u) ? c.lag[1] : e_yp) - ((b & 4u) ? c.lag[1] : e_yn);
+        const double dz_ = ((b & 32u) ? c.lag[2] : e_zp) - ((b & 16u) ? c.lag[2] : e_zn);
+        c.lag[0] = (b & 1u) ? e_xn : e_xp;
+        c.lag[1] = (b & 4u) ? e_yn : e_yp;
+        c.lag[2] = (b & 16u) ? e_zn : e_zp;
+        const double ex = e_xn + e_xp, ey = e_yn + e_yp, ez = e_zn + e_zp;
+        double e_new = next<true>(c, dx_, dy_, dz_, ex, ey, ez);
+        if (!(fabs(e_new) < 1.0e300)) e_new = next<false>(c, dx_, dy_, dz_, ex, ey, ez);
+        if (b & WALL) e_new = e;
+        if (b & ABOVE) e_new = e_zn + dp_dz;
+        if (!(b & FREE)) return e;
+        if (check) {
+            const double norm = (e_new - e) * (e_new - e) / (e_new * e_new + 1.0e-16);
+            bits = (unsigned long long)__double_as_longlong(fabs(norm));
+        }
+        return e * (1.0 - q.theta) + e_new * q.theta;
+    }
+    // as k_ns_decide
+    __device__ unsigned verdict(unsigned long long m, unsigned) const
+    {
+        const double v = __longlong_as_double((long long)m);
+        return v != v ? 2u : v < tolerance ? 1u : 0u;
+    }
+    __device__ void record(unsigned long long m, unsigned it, unsigned verdict) const
+    {
+        st->lastmax = m;
+        if (verdict == 1u) st->conv_nijac = it;
+        if (verdict) atomicMax(&st->done, verdict);
+    }
+    __device__ void finish(int x, int y, int z, double value, double previous) const
+    {
+        B[cidx(g, x, y, z)] = value;
+        ghost_cell_writes(g, x, y, z, previous, B);
+    }
+};
 
 // smoothing<Float>, src/navierstokes.cuh:2619-2677, A -> B (all interior
 // cells written; ghosts follow from a ghost pass)
@@ -698,6 +824,9 @@ struct sph_ns {
     int cur = 0;
     long iter = 0;
     double t = 0.0;
+    Resident res;           // tiles and inboxes of the resident iterations
+    uint32_t res_spin = 0;  // their wait bound in polls (0: the default)
+    double *eps_start = nullptr;  // a solve's start, where it takes several of their launches
     sph_ns_stats st{};
 };
 
@@ -755,6 +884,71 @@ int read_state(sph_ns *n)
     return hip_ok(hipStreamSynchronize(n->s), "Navier-Stokes Jacobi iterations");
 }
 
+// The Jacobi iterations of a solve in resident launches, each from
+// eps[cur] into the other buffer.  With resident = false on return a wait
+// ran out: the iterate is back at the solve's start, and this fluid goes on
+// with one launch per iteration.
+int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
+{
+    const sph_ns_params &P = n->P;
+    const NsGrid &g = n->g;
+    const unsigned chunk = 20000u;  // iterations of a launch: some 30 ms
+    const bool keep = P.maxiter > chunk;
+    if (keep && !n->eps_start &&
+        hipMalloc((void **)&n->eps_start, n->nc * sizeof(double)) != hipSuccess) {
+        n->eps_start = nullptr;
+        (void)hipGetLastError();
+        resident = false;
+        return SPH_OK;
+    }
+    int rc = SPH_OK;
+    const double dxdx = g.dx * g.dx, dydy = g.dy * g.dy, dzdz = g.dz * g.dz;
+    double *start = n->eps[n->cur];
+    if (keep) {
+        rc = hip_ok(hipMemcpyAsync(n->eps_start, start, n->nc * sizeof(double), hipMemcpyDeviceToDevice, n->s),
+                    "hipMemcpyAsync");
+        if (rc) return rc;
+    }
+    const int cur0 = n->cur;
+    for (unsigned it = 0; it < P.maxiter; it += std::min(chunk, P.maxiter - it)) {
+        ResidentArgs a;
+        bool ok = resident_args(n->res, n->s, g.nx, g.ny, g.nz, it, it + std::min(chunk, P.maxiter - it),
+                                n->res_spin, a);
+        if (ok) {
+            const NsOp op{g, n->q, n->eps[n->cur], n->eps[1 - n->cur], cv(n->vp), cv(n->vpf), n->phi, n->dphi,
+                          n->dst, P.tolerance, n->dp_dz, n->wall0_iz, fixed_div(2.0 * g.dx),
+                          fixed_div(2.0 * g.dy), fixed_div(2.0 * g.dz),
+                          fixed_div(2.0 * (dxdx * dydy + dxdx * dzdz + dydy * dzdz))};
+            resident_launch(n->res, n->device, n->s, a, op);
+            rc = hip_ok(hipGetLastError(), "Navier-Stokes resident iterations");
+            if (!rc) rc = read_state(n);
+            if (rc) return rc;
+            ok = n->hst->done != RES_ABORT;
+        }
+        if (!ok) {
+            n->res.usable = false;
+            resident = false;
+            n->cur = cur0;
+            rc = hip_ok(hipMemsetAsync(n->dst, 0, sizeof(NsSolveState), n->s), "hipMemsetAsync");
+            if (!rc && it > 0)
+                rc = hip_ok(hipMemcpyAsync(start, n->eps_start, n->nc * sizeof(double),
+                                           hipMemcpyDeviceToDevice, n->s), "hipMemcpyAsync");
+            return rc;
+        }
+        if (n->hst->done == 2u) {
+            n->cur = cur0;
+            return fail(SPH_ERR_NAN, "normalized residual is NaN");
+        }
+        n->cur = 1 - n->cur;
+        if (n->hst->done == 1u) {
+            converged = true;
+            break;
+        }
+    }
+    nijac = converged ? n->hst->conv_nijac + 1 : P.maxiter;
+    return SPH_OK;
+}
+
 // One fluid solve, src/device.cu:1354-1898
 int ns_solve(sph_ns *n)
 {
@@ -803,30 +997,42 @@ int ns_solve(sph_ns *n)
     int rc = hip_ok(hipMemsetAsync(n->dst, 0, sizeof(NsSolveState), n->s), "hipMemsetAsync");
     if (rc) return rc;
     const int cur0 = n->cur;
-    unsigned next = 0;
     bool converged = false;
-    while (next < P.maxiter) {
-        const unsigned last = std::min<unsigned>(P.maxiter - 1, (next + 99) / 10 * 10);
-        for (unsigned it = next; it <= last; ++it) {
-            const int check = it % 10 == 0;
-            const int a = cur0 ^ (int)(it & 1u);
-            hipLaunchKernelGGL(k_ns_jacobi, dim3(cb), dim3(NS_THREADS), 0, n->s, g, n->q, it, n->eps[a],
-                               n->eps[1 - a], n->f1, n->f2, cv(n->vp), cv(n->vpf), n->phi, n->dphi, n->dst,
-                               check, n->wall0_iz, n->dp_dz);
-            if (check)
-                hipLaunchKernelGGL(k_ns_decide, dim3(1), dim3(64), 0, n->s, n->dst, it, P.tolerance);
-        }
-        next = last + 1;
-        rc = read_state(n);
+    unsigned nijac = 0;
+    // A ghost layer that no rule writes (one z boundary periodic, the other
+    // not) keeps a different value in each buffer: one launch per iteration
+    if (!n->res.planned)
+        resident_plan(n->res, n->device, g.nx, g.ny, g.nz, 3 | (g.bb == 2 && g.bt == 2 ? 4 : 0));
+    bool resident = n->res.usable && (g.bb == 2) == (g.bt == 2);
+    if (resident) {
+        rc = ns_resident(n, resident, converged, nijac);
         if (rc) return rc;
-        if (n->hst->done == 2u) return fail(SPH_ERR_NAN, "normalized residual is NaN");
-        if (n->hst->done == 1u) {
-            converged = true;
-            break;
-        }
     }
-    const unsigned nijac = converged ? n->hst->conv_nijac + 1 : P.maxiter;
-    n->cur = cur0 ^ (int)(nijac & 1u);
+    if (!resident) {
+        unsigned next = 0;
+        while (next < P.maxiter) {
+            const unsigned last = std::min<unsigned>(P.maxiter - 1, (next + 99) / 10 * 10);
+            for (unsigned it = next; it <= last; ++it) {
+                const int check = it % 10 == 0;
+                const int a = cur0 ^ (int)(it & 1u);
+                hipLaunchKernelGGL(k_ns_jacobi, dim3(cb), dim3(NS_THREADS), 0, n->s, g, n->q, it, n->eps[a],
+                                   n->eps[1 - a], n->f1, n->f2, cv(n->vp), cv(n->vpf), n->phi, n->dphi, n->dst,
+                                   check, n->wall0_iz, n->dp_dz);
+                if (check)
+                    hipLaunchKernelGGL(k_ns_decide, dim3(1), dim3(64), 0, n->s, n->dst, it, P.tolerance);
+            }
+            next = last + 1;
+            rc = read_state(n);
+            if (rc) return rc;
+            if (n->hst->done == 2u) return fail(SPH_ERR_NAN, "normalized residual is NaN");
+            if (n->hst->done == 1u) {
+                converged = true;
+                break;
+            }
+        }
+        nijac = converged ? n->hst->conv_nijac + 1 : P.maxiter;
+        n->cur = cur0 ^ (int)(nijac & 1u);
+    }
     double max_norm;
     std::memcpy(&max_norm, &n->hst->lastmax, sizeof max_norm);
     n->st.solves++;
@@ -910,9 +1116,11 @@ int ensure_force_rows(sph_ns *n, uint32_t np)
 
 int ns_coupled_step(sph_ns *n, uint32_t np, const double *x, const double *vel, const double *xs,
                     const uint32_t *cstart, const uint32_t *cend, const uint32_t *gidx,
-                    const double *origo, int periodic, double *force, double wall_x, hipStream_t s)
+                    const double *origo, int periodic, double *force, double wall_x, uint32_t spin,
+                    hipStream_t s)
 {
     n->wall_x = wall_x;
+    n->res_spin = spin;
     // the fluid's launches go on the context's stream, after its forces
     hipStream_t own = n->s;
     n->s = s;
@@ -1071,6 +1279,8 @@ void sph_ns_destroy(sph_ns *n)
     if (n->arena) hipFree(n->arena);
     if (n->grains) hipFree(n->grains);
     if (n->own_forces) hipFree(n->own_forces);
+    if (n->eps_start) hipFree(n->eps_start);
+    resident_free(n->res);
     if (n->hst) hipHostFree(n->hst);
     if (n->s) hipStreamDestroy(n->s);
     delete n;
