@@ -728,9 +728,10 @@ __device__ bool grid_scan(uint32_t *__restrict__ a, uint32_t m, uint32_t *__rest
     return true;
 }
 
-// Block `bid` of the G blocks that rebuild one box.
+// Block `bid` of the G blocks that rebuild one box; l: the list build that
+// follows in the same launch, or none.
 __device__ __forceinline__ void rebuild_body(const StepArgs &a, const RebuildArgs &r, uint32_t bid,
-                                             uint32_t G)
+                                             uint32_t G, const NlBuildTask *l = nullptr)
 {
     if ((*r.cond & NLF_REBUILD) == 0u) return;
     if ((*r.err & ERRF_BARRIER) != 0u) return;  // an earlier barrier timed out
@@ -774,6 +775,16 @@ __device__ __forceinline__ void rebuild_body(const StepArgs &a, const RebuildArg
         r.vel_s[idx] = r.vel[sidx];
         r.angvel_s[idx] = r.angvel[sidx];
     }
+    if (!l || !grid_barrier(r.bar, G, gen, r.err, r.spin_limit)) return;
+    nl_build_body(l->a, l->n, l->cond, l->vals, l->cell_start, l->cell_end, l->x_s, l->nl, l->nl_cnt,
+                  l->nl_pos, l->x_ref, l->flags, l->contacts, l->cmask, l->nl_slot, l->slot_cand,
+                  l->nl_gap, l->nl_gmin, l->err, bid, G);
+}
+
+// Sort, reorder and list build of a small box in one launch.
+__global__ void __launch_bounds__(256) k_rebuild_lists(RebuildArgs r, NlBuildTask l)
+{
+    rebuild_body(l.a, r, blockIdx.x, gridDim.x, &l);
 }
 
 __global__ void __launch_bounds__(256) k_rebuild(StepArgs a, RebuildArgs r)
@@ -781,12 +792,14 @@ __global__ void __launch_bounds__(256) k_rebuild(StepArgs a, RebuildArgs r)
     rebuild_body(a, r, blockIdx.x, gridDim.x);
 }
 
+#define REBUILD_LISTS 2u
 int rebuild_blocks_per_cu()
 {
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rebuild, 256, 0) != hipSuccess)
+    int nb = 0, nl = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_rebuild, 256, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nl, k_rebuild_lists, 256, 0) != hipSuccess)
         return 0;
-    return nb;
+    return nb < nl ? nb : nl;
 }
 
 void launch_rebuild(hipStream_t s, const StepArgs &a, const NLArgs &n, DemBuffers &b,
@@ -795,7 +808,17 @@ void launch_rebuild(hipStream_t s, const StepArgs &a, const NLArgs &n, DemBuffer
 {
     if (a.np == 0) return;
     const RebuildTask t = rebuild_task(a, b, ncells, bits, cond, spin_limit);
-    hipLaunchKernelGGL(k_rebuild, dim3(blocks), dim3(256), 0, s, t.a, t.r);
+    // A launch that returns at once costs a small box 5% of its step: where
+    // the list build takes each thread at most REBUILD_LISTS grains, it joins.
+    const bool joined = a.np <= REBUILD_LISTS * 256u * blocks;
+    if (joined) {
+        DemBuffers sorted = b;  // the lists read the buffer the last pass writes
+        if (t.r.passes & 1u) sorted.vals = b.vals_tmp;
+        hipLaunchKernelGGL(k_rebuild_lists, dim3(blocks), dim3(256), 0, s, t.r,
+                           nl_build_task(a, n, sorted, cond));
+    } else {
+        hipLaunchKernelGGL(k_rebuild, dim3(blocks), dim3(256), 0, s, t.a, t.r);
+    }
     // the sorted keys and values end in the buffer the last pass wrote
     if (t.r.passes & 1u) {
         uint32_t *tk = b.keys;
@@ -805,6 +828,7 @@ void launch_rebuild(hipStream_t s, const StepArgs &a, const NLArgs &n, DemBuffer
         b.vals = b.vals_tmp;
         b.vals_tmp = tv;
     }
+    if (joined) return;
     // the list build, the heaviest phase, on one thread per grain (it
     // needs no barrier after it, so its grid is not bounded by residency)
     const NlBuildTask l = nl_build_task(a, n, b, cond);
@@ -1459,6 +1483,73 @@ __device__ void owner_test_all(const Grid &g, uint32_t np, uint32_t pos, uint32_
     }
 }
 
+// Left-to-right sum part[0] + part[1] + ... (the reference's serial loop,
+// src/integration.cuh:361-364) by one wave, every lane holding the result.
+// Terms equal to +0.0 are skipped (serial_sum_staged says why that is exact):
+// 512 partials in registers at a time, the non-zero ones found by ballot and
+// added in order from their lanes.
+__device__ __forceinline__ double serial_sum_wave(const double *__restrict__ part, uint32_t n)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    double s = 0.0;
+    for (uint32_t base = 0; base < n; base += 512u) {
+        double v[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            const uint32_t j = base + 64u * u + lane;
+            v[u] = j < n ? part[j] : 0.0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            const long long b = __double_as_longlong(v[u]);
+            unsigned long long nz = __ballot(b != 0ll);
+            while (nz) {
+                const int l = __ffsll(nz) - 1;
+                nz &= nz - 1ull;
+                const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)b, l);
+                const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), l);
+                s += __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+            }
+        }
+    }
+    return s;
+}
+
+// The end of a step, by one wave: integrateWalls (src/integration.cuh:344-450;
+// the serial sum over the block partials in the reference's order, formed once
+// where the reference sums wall 0's partials for each wall), then the host's
+// time loop update of the clock (iter += 1, time += dt, src/device.cu:2541-2545).
+__device__ __forceinline__ void step_end_wave(const StepArgs &a, const StepEnd &w)
+{
+    const long long iter = w.clock->iter;
+    const double t_current = w.clock->time;
+    const uint32_t idx = threadIdx.x & 63u;
+    if (a.walls.nw > 0) {
+        const double total = serial_sum_wave(w.partial, w.nparts);
+        const int wmode = idx < a.walls.nw ? a.walls.wmode[idx] : 0;
+        if (wmode != 0) {
+            double4 nx = w.w_nx[idx], mvfd = w.w_mvfd[idx];
+            const double dt = a.dt;
+            double acc0 = iter == 0 ? 0.0 : w.w_acc[idx];
+            mvfd.z = total;
+            const double sigma_0 = mvfd.w + a.prm.sigma0_A * sin(2.0 * PI_REF * a.prm.sigma0_f * t_current);
+            const double N = -sigma_0 * a.grid.L[0] * a.grid.L[1];
+            double acc = (mvfd.z + N) / mvfd.x;
+            if (wmode == 2) acc = 0.0;
+            const double dacc_dt = (acc - acc0) / dt;
+            nx.w += mvfd.y * dt + 0.5 * acc * dt * dt + 1.0 / 6.0 * dacc_dt * dt * dt * dt;
+            mvfd.y += acc * dt + 0.5 * dacc_dt * dt * dt;
+            w.w_nx[idx] = nx;
+            w.w_mvfd[idx] = mvfd;
+            w.w_acc[idx] = acc;
+        }
+    }
+    if (idx == 0) {
+        w.clock->iter = iter + 1;
+        w.clock->time = t_current + a.dt;
+    }
+}
+
 #define TW 64
 #define TU 4
 // NEAR: grid searched one cell deep (nearest_image applies; the cell code of
@@ -1686,11 +1777,18 @@ __global__ void __launch_bounds__(TW) k_topology_lists(
     uint8_t *__restrict__ slot_cand, const uint32_t *__restrict__ nl_cnt,
     const uint32_t *__restrict__ nl_pos, const uint32_t *__restrict__ cellc,
     const float *__restrict__ nl_gap, const float *__restrict__ nl_gmin,
-    const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur)
+    const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur,
+    StepEnd end)
 {
+    // The end of the step before: the first block of eight, so that the
+    // search's blocks keep their XCDs (blocks are dealt to them mod 8).
+    if (blockIdx.x < 8u) {
+        if (blockIdx.x == 0u && end.clock) step_end_wave(a, end);
+        return;
+    }
     topology_lists_body<NEAR>(a, vals, cell_start, cell_end, x, x_s, contacts, cmask, err, nl,
                               nl_slot, slot_cand, nl_cnt, nl_pos, cellc, nl_gap, nl_gmin, nl_disp,
-                              flags_rw, cur, blockIdx.x, gridDim.x);
+                              flags_rw, cur, blockIdx.x - 8u, gridDim.x - 8u);
 }
 
 // Wall contacts of one particle, contactsearch.cuh:420-701: the top wall
@@ -2028,21 +2126,23 @@ __global__ void __launch_bounds__(256) k_contact_viscous(
 }
 
 void launch_topology(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool nlist,
-                     bool near, uint32_t cur)
+                     bool near, uint32_t cur, bool end)
 {
     if (a.prm.contactmodel == 1) return;  // model 1 keeps no contact history
     if (nlist) {
         const TopoTask t = topology_task(a, b, cur);
+        const uint32_t nw = 8u + (a.np + 63u) / 64u;
+        const StepEnd e = end ? step_end(a, b) : StepEnd{};
         if (near)
-            hipLaunchKernelGGL(k_topology_lists<true>, dim3(topology_blocks(a.np)), dim3(TW), 0, s,
+            hipLaunchKernelGGL(k_topology_lists<true>, dim3(nw), dim3(TW), 0, s,
                                t.a, t.vals, t.cell_start, t.cell_end, t.x, t.x_s, t.contacts,
                                t.cmask, t.err, t.nl, t.nl_slot, t.slot_cand, t.nl_cnt, t.nl_pos,
-                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur);
+                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, e);
         else
-            hipLaunchKernelGGL(k_topology_lists<false>, dim3(topology_blocks(a.np)), dim3(TW), 0,
-                               s, t.a, t.vals, t.cell_start, t.cell_end, t.x, t.x_s, t.contacts,
+            hipLaunchKernelGGL(k_topology_lists<false>, dim3(nw), dim3(TW), 0, s,
+                               t.a, t.vals, t.cell_start, t.cell_end, t.x, t.x_s, t.contacts,
                                t.cmask, t.err, t.nl, t.nl_slot, t.slot_cand, t.nl_cnt, t.nl_pos,
-                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur);
+                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, e);
     } else
         hipLaunchKernelGGL(k_topology_cells, dim3((a.np + 255) / 256), dim3(256), 0, s, a,
                            b.vals, b.cell_start, b.cell_end, b.x_s, b.contacts, b.cmask,
@@ -2059,7 +2159,7 @@ void launch_contact(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool 
         return;
     }
     const ForcesTask t = forces_task(a, b, nlist);
-    const uint32_t nw = forces_blocks(a.np);
+    const uint32_t nw = (a.np + 63u) / 64u;
     if (a.prm.contactmodel == 3)
         hipLaunchKernelGGL(k_forces<true>, dim3(nw), dim3(FW), 0, s, t.a, t.order, t.x, t.vel,
                            t.angvel, t.force, t.torque, t.es_dot, t.ev_dot, t.es, t.ev, t.p,
@@ -2497,69 +2597,13 @@ void launch_integrate(hipStream_t s, const StepArgs &a, const DemBuffers &b,
                        t.tau_eff, t.walls_force_pp, t.wall_partial, t.bg, t.nh);
 }
 
-// integrateWalls, src/integration.cuh:344-450.  One wave: lane 0 forms the
-// serial sum over the block partials (the reference's order) once and every
-// wall thread uses it (the reference sums wall 0's partials for each wall).
-__device__ __forceinline__ void integrate_walls_body(
-    const StepArgs &a, const StepClock *__restrict__ clock, double4 *__restrict__ w_nx,
-    double4 *__restrict__ w_mvfd, double *__restrict__ w_acc,
-    const double *__restrict__ partial, uint32_t nparts)
+__global__ void __launch_bounds__(64) k_step_end(StepArgs a, StepEnd w) { step_end_wave(a, w); }
+
+void launch_step_end(hipStream_t s, const StepArgs &a, const DemBuffers &b)
 {
-    const long long iter = clock->iter;
-    const double t_current = clock->time;
-    __shared__ double lds[SUM_CHUNK];
-    __shared__ double total;
-    const double s = serial_sum_staged(partial, nparts, lds);
-    if (threadIdx.x == 0) total = s;
-    __syncthreads();
-    uint32_t idx = threadIdx.x;
-    if (idx >= a.walls.nw) return;
-    int wmode = a.walls.wmode[idx];
-    if (wmode == 0) return;
-    double4 nx = w_nx[idx], mvfd = w_mvfd[idx];
-    const double dt = a.dt;
-    double acc0 = iter == 0 ? 0.0 : w_acc[idx];
-    mvfd.z = total;
-    const double sigma_0 = mvfd.w + a.prm.sigma0_A * sin(2.0 * PI_REF * a.prm.sigma0_f * t_current);
-    const double N = -sigma_0 * a.grid.L[0] * a.grid.L[1];
-    double acc = (mvfd.z + N) / mvfd.x;
-    if (wmode == 2) acc = 0.0;
-    const double dacc_dt = (acc - acc0) / dt;
-    nx.w += mvfd.y * dt + 0.5 * acc * dt * dt + 1.0 / 6.0 * dacc_dt * dt * dt * dt;
-    mvfd.y += acc * dt + 0.5 * dacc_dt * dt * dt;
-    w_nx[idx] = nx;
-    w_mvfd[idx] = mvfd;
-    w_acc[idx] = acc;
+    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(64), 0, s, a, step_end(a, b));
 }
 
-__global__ void __launch_bounds__(SUM_THREADS) k_integrate_walls(
-    StepArgs a, const StepClock *__restrict__ clock, double4 *__restrict__ w_nx,
-    double4 *__restrict__ w_mvfd, double *__restrict__ w_acc,
-    const double *__restrict__ partial, uint32_t nparts)
-{
-    integrate_walls_body(a, clock, w_nx, w_mvfd, w_acc, partial, nparts);
-}
-
-void launch_integrate_walls(hipStream_t s, const StepArgs &a, const DemBuffers &b)
-{
-    const WallsTask t = walls_task(a, b);
-    hipLaunchKernelGGL(k_integrate_walls, dim3(1), dim3(SUM_THREADS), 0, s, t.a, t.clock, t.w_nx,
-                       t.w_mvfd, t.w_acc, t.partial, t.nparts);
-}
-
-// iter += 1, time += dt: the host's time loop update (src/device.cu:2541-2545)
-__global__ void k_clock_advance(StepClock *__restrict__ clock, double dt)
-{
-    if (threadIdx.x == 0) {
-        clock->iter += 1;
-        clock->time += dt;
-    }
-}
-
-void launch_clock_advance(hipStream_t s, StepClock *clock, double dt)
-{
-    hipLaunchKernelGGL(k_clock_advance, dim3(1), dim3(64), 0, s, clock, dt);
-}
 
 // ------------------------------------------------------------------
 // helpers
@@ -2782,17 +2826,16 @@ IntegrateTask integrate_task(const StepArgs &a, const DemBuffers &b, int change_
     return t;
 }
 
-WallsTask walls_task(const StepArgs &a, const DemBuffers &b)
+StepEnd step_end(const StepArgs &a, const DemBuffers &b)
 {
-    WallsTask t;
-    t.a = a;
-    t.clock = b.clock;
-    t.w_nx = b.w_nx;
-    t.w_mvfd = b.w_mvfd;
-    t.w_acc = b.w_acc;
-    t.partial = b.wall_partial;
-    t.nparts = (a.np + 255) / 256;
-    return t;
+    StepEnd e;
+    e.clock = b.clock;
+    e.w_nx = b.w_nx;
+    e.w_mvfd = b.w_mvfd;
+    e.w_acc = b.w_acc;
+    e.partial = b.wall_partial;
+    e.nparts = (a.np + 255) / 256;
+    return e;
 }
 
 uint32_t topology_blocks(uint32_t np) { return (np + TW - 1) / TW; }
@@ -2862,19 +2905,9 @@ __global__ void __launch_bounds__(256) k_integrate_multi(const IntegrateTask *__
                    T.tau_eff, T.walls_force_pp, T.wall_partial, T.bg, T.nh, bid);
 }
 
-__global__ void __launch_bounds__(SUM_THREADS) k_walls_multi(const WallsTask *__restrict__ t)
+__global__ void __launch_bounds__(64) k_step_end_multi(const StepEndTask *__restrict__ t)
 {
-    const WallsTask &T = t[blockIdx.x];
-    integrate_walls_body(T.a, T.clock, T.w_nx, T.w_mvfd, T.w_acc, T.partial, T.nparts);
-}
-
-__global__ void k_clock_multi(const ClockTask *__restrict__ t, uint32_t n)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) {
-        t[k].clock->iter += 1;
-        t[k].clock->time += t[k].dt;
-    }
+    step_end_wave(t[blockIdx.x].a, t[blockIdx.x].e);
 }
 
 void launch_rebuild_multi(hipStream_t s, const RebuildTask *t, MultiMap m, uint32_t blocks)
@@ -2975,12 +3008,7 @@ void launch_bond_gather_multi(hipStream_t s, const BondGatherTask *t, MultiMap m
     if (blocks) hipLaunchKernelGGL(k_bond_gather_multi, dim3(blocks), dim3(256), 0, s, t, m);
 }
 
-void launch_walls_multi(hipStream_t s, const WallsTask *t, uint32_t n)
+void launch_step_end_multi(hipStream_t s, const StepEndTask *t, uint32_t n)
 {
-    if (n) hipLaunchKernelGGL(k_walls_multi, dim3(n), dim3(SUM_THREADS), 0, s, t);
-}
-
-void launch_clock_multi(hipStream_t s, const ClockTask *t, uint32_t n)
-{
-    if (n) hipLaunchKernelGGL(k_clock_multi, dim3((n + 63) / 64), dim3(64), 0, s, t, n);
+    if (n) hipLaunchKernelGGL(k_step_end_multi, dim3(n), dim3(64), 0, s, t);
 }

@@ -43,11 +43,10 @@ struct sph_ctx {
     int device = 0;
     sph_ns *ns = nullptr;  // an attached Navier-Stokes fluid (sph_ns_attach)
     hipStream_t stream = nullptr;
-    // integrateWalls runs on `aux`, overlapped with the next step's contact
-    // search (which does not read the walls); the contact forces wait for it
-    hipStream_t aux = nullptr;
-    hipEvent_t ev_integrated = nullptr, ev_walls = nullptr;
-    bool walls_pending = false;
+    // the last step's wall integration and clock advance are still to be
+    // launched: the next step's contact search, which reads neither, takes
+    // them along, and finish_step() launches them otherwise
+    bool end_pending = false;
     std::string err;
     bool loaded = false;
     uint64_t gen = 0;  // incremented by every load (captured graphs hold the old buffers)
@@ -174,23 +173,24 @@ static void prof_flush(sph_ctx *ctx)
     ctx->ev_used = 0;
 }
 
-// The main stream waits for the pending wall update (work enqueued after
-// this sees the new wall state).
-static int wait_walls(sph_ctx *ctx)
+static StepArgs step_args(const sph_ctx *ctx);
+
+// The end of the last step, where no search took it along.
+static int finish_step(sph_ctx *ctx)
 {
-    if (ctx->walls_pending) {
-        HIPCHK(hipStreamWaitEvent(ctx->stream, ctx->ev_walls, 0));
-        ctx->walls_pending = false;
+    if (ctx->end_pending) {
+        ctx->end_pending = false;
+        ProfScope ps(ctx, SPH_K_WALLS);
+        launch_step_end(ctx->stream, step_args(ctx), ctx->db);
     }
     return SPH_OK;
 }
 
 static int sync(sph_ctx *ctx)
 {
-    int rc = wait_walls(ctx);
+    int rc = finish_step(ctx);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->aux));
     HIPCHK(hipGetLastError());
     if (ctx->prof) prof_flush(ctx);
     return SPH_OK;
@@ -248,8 +248,7 @@ static void free_device(sph_ctx *ctx)
 {
     net_release(ctx);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->aux) (void)hipStreamSynchronize(ctx->aux);
-    ctx->walls_pending = false;
+    ctx->end_pending = false;
     resident_free(ctx->res);
     for (void *p : ctx->allocs) (void)hipFree(p);
     ctx->allocs.clear();
@@ -1269,7 +1268,7 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
     int rc;
     if (h.np > 0) {
         if (h.adaptive == 1 && h.nw > 0) {  // updateGridSize, device.cu:370-400
-            rc = wait_walls(ctx);
+            rc = finish_step(ctx);
             if (rc) return rc;
             HIPCHK(hipMemcpyAsync(ctx->h_d, (const char *)ctx->db.w_nx + 24, 8,
                                   hipMemcpyDeviceToHost, s));
@@ -1299,9 +1298,8 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
                 { ProfScope ps(ctx, SPH_K_NLIST); launch_nl_build(s, a, ctx->nla, ctx->db, cond); }
             }
             { ProfScope ps(ctx, SPH_K_TOPOLOGY);
-              launch_topology(s, a, ctx->db, true, ctx->nla.range == 1, cur); }
-            rc = wait_walls(ctx);
-            if (rc) return rc;
+              launch_topology(s, a, ctx->db, true, ctx->nla.range == 1, cur, ctx->end_pending); }
+            ctx->end_pending = false;
             { ProfScope ps(ctx, SPH_K_CONTACT); launch_contact(s, a, ctx->db, true); }
             ctx->nl_parity ^= 1u;
             ctx->nl_force = 0;
@@ -1313,7 +1311,7 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
                 ProfScope ps(ctx, SPH_K_TOPOLOGY);
                 launch_topology(s, a, ctx->db, false, false, 0u);
             }
-            rc = wait_walls(ctx);
+            rc = finish_step(ctx);
             if (rc) return rc;
             { ProfScope ps(ctx, SPH_K_CONTACT); launch_contact(s, a, ctx->db, false); }
         }
@@ -1365,22 +1363,13 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
           launch_integrate(s, a, ctx->db, change_velocity_state, 10.0, h.tau_x,
                            gather_in_integrate(ctx), nh); }
         ctx->hash_ready = fuse_hash;
-        if (h.nw > 0) {
-            HIPCHK(hipEventRecord(ctx->ev_integrated, s));
-            HIPCHK(hipStreamWaitEvent(ctx->aux, ctx->ev_integrated, 0));
-            {
-                ProfScope ps(ctx, SPH_K_WALLS, ctx->aux);
-                launch_integrate_walls(ctx->aux, a, ctx->db);
-            }
-            // the clock's last readers this step are integrate and the walls
-            launch_clock_advance(ctx->aux, ctx->db.clock, h.time_dt);
-            HIPCHK(hipEventRecord(ctx->ev_walls, ctx->aux));
-            ctx->walls_pending = true;
-        } else {
-            launch_clock_advance(s, ctx->db.clock, h.time_dt);
+        ctx->end_pending = true;
+        if (ctx->prof) {
+            rc = finish_step(ctx);
+            if (rc) return rc;
         }
     } else if (ctx->db.clock) {
-        launch_clock_advance(s, ctx->db.clock, h.time_dt);
+        launch_step_end(s, step_args(ctx), ctx->db);
     }
     h.time_current += h.time_dt;
     ctx->filetimeclock += h.time_dt;
@@ -1417,9 +1406,6 @@ sph_ctx *sph_create(int device)
     sph_ctx *ctx = new sph_ctx();
     ctx->device = device;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->ev_integrated, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->ev_walls, hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc((void **)&ctx->h_err, 128, hipHostMallocDefault) != hipSuccess) {
         g_last_error = "stream or pinned allocation failed";
         delete ctx;
@@ -1462,10 +1448,7 @@ void sph_destroy(sph_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     free_device(ctx);
     for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
-    if (ctx->ev_integrated) (void)hipEventDestroy(ctx->ev_integrated);
-    if (ctx->ev_walls) (void)hipEventDestroy(ctx->ev_walls);
     if (ctx->h_err) (void)hipHostFree(ctx->h_err);
-    if (ctx->aux) (void)hipStreamDestroy(ctx->aux);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -2019,18 +2002,14 @@ struct EnsStage {
 
 struct EnsPhase {  // the launches of one step
     EnsStage rebuild, nlbuild, topo[2], forces[2], bonds, integ;
-    void *walls = nullptr;
-    uint32_t nwalls = 0;
-    void *clocks = nullptr;
-    uint32_t nclocks = 0;
+    void *ends = nullptr;
+    uint32_t nends = 0;
 };
 
 struct EnsFluidPhase {  // the particle-side launches of one step of the fluid boxes
     EnsStage hash, rebuild, nlbuild, topo[2], forces[2], bonds, gather, integ;
-    void *walls = nullptr;
-    uint32_t nwalls = 0;
-    void *clocks = nullptr;
-    uint32_t nclocks = 0;
+    void *ends = nullptr;
+    uint32_t nends = 0;
 };
 
 struct sph_ensemble {
@@ -2216,8 +2195,7 @@ static int ens_plan(sph_ensemble *e)
         std::vector<ForcesTask> frc[2];
         std::vector<BondTask> bnd;
         std::vector<IntegrateTask> itg;
-        std::vector<WallsTask> wls;
-        std::vector<ClockTask> clk;
+        std::vector<StepEndTask> end;
         std::vector<uint32_t> n_rb, n_nlb, n_topo[2], n_frc[2], n_bnd, n_itg;
         for (size_t i = 0; i < e->multi.size(); ++i) {
             const sph_ctx *c = e->boxes[e->multi[i]];
@@ -2260,8 +2238,7 @@ static int ens_plan(sph_ensemble *e)
             nh.disp2 = c->nla.disp2;
             itg.push_back(integrate_task(a, b, 0, 10.0, h.tau_x, true, nh));
             n_itg.push_back((h.np + 255) / 256);
-            if (h.nw > 0) wls.push_back(walls_task(a, b));
-            clk.push_back(ClockTask{b.clock, h.time_dt});
+            end.push_back(StepEndTask{a, step_end(a, b)});
         }
         EnsPhase &P = e->ph[j];
         int rc;
@@ -2271,15 +2248,14 @@ static int ens_plan(sph_ensemble *e)
             (rc = ens_stage(e, P.forces[0], frc[0], n_frc[0])) ||
             (rc = ens_stage(e, P.forces[1], frc[1], n_frc[1])) ||
             (rc = ens_stage(e, P.bonds, bnd, n_bnd)) || (rc = ens_stage(e, P.integ, itg, n_itg)) ||
-            (rc = ens_array(e, P.walls, wls)) || (rc = ens_array(e, P.clocks, clk)))
+            (rc = ens_array(e, P.ends, end)))
             return rc;
-        P.nwalls = (uint32_t)wls.size();
-        P.nclocks = (uint32_t)clk.size();
+        P.nends = (uint32_t)end.size();
         if (j == 0) {
             const EnsStage *all[] = {&P.rebuild, &P.nlbuild, &P.topo[0], &P.topo[1], &P.forces[0],
                                      &P.forces[1], &P.bonds, &P.integ};
             for (const EnsStage *st : all) e->launches_per_step += st->blocks ? 1u : 0u;
-            e->launches_per_step += (P.nwalls ? 1u : 0u) + (P.nclocks ? 1u : 0u);
+            e->launches_per_step += P.nends ? 1u : 0u;
         }
     }
     e->planned = true;
@@ -2319,8 +2295,7 @@ static void ens_enqueue_phase(sph_ensemble *e, const EnsPhase &P)
     launch_forces_multi(s, (const ForcesTask *)P.forces[1].tasks, mm(P.forces[1]), P.forces[1].blocks, true);
     launch_bonds_multi(s, (const BondTask *)P.bonds.tasks, mm(P.bonds), P.bonds.blocks);
     launch_integrate_multi(s, (const IntegrateTask *)P.integ.tasks, mm(P.integ), P.integ.blocks);
-    launch_walls_multi(s, (const WallsTask *)P.walls, P.nwalls);
-    launch_clock_multi(s, (const ClockTask *)P.clocks, P.nclocks);
+    launch_step_end_multi(s, (const StepEndTask *)P.ends, P.nends);
 }
 
 // The host side of one step of a multi-box box (what step_once changes).
@@ -2432,7 +2407,7 @@ int sph_ensemble_autotune(sph_ensemble *e, int trial_steps, const double *fracti
                 for (int s = 0; s < trial_steps && !rc; ++s)
                     rc = step_once(c, nullptr, nullptr, std::string());
                 if (rc) break;
-                if ((rc = wait_walls(c))) break;
+                if ((rc = finish_step(c))) break;
                 float el = 0.0f;
                 if (hipEventRecord(t1, c->stream) != hipSuccess || hipEventSynchronize(t1) != hipSuccess ||
                     hipEventElapsedTime(&el, t0, t1) != hipSuccess) { rc = SPH_ERR_HIP; break; }
@@ -2569,8 +2544,7 @@ static int ens_fluid_plan(sph_ensemble *e)
         std::vector<BondTask> bnd;
         std::vector<BondGatherTask> bgt;
         std::vector<IntegrateTask> itg;
-        std::vector<WallsTask> wls;
-        std::vector<ClockTask> clk;
+        std::vector<StepEndTask> end;
         std::vector<uint32_t> n_hs, n_rb, n_nlb, n_topo[2], n_frc[2], n_bnd, n_bgt, n_itg;
         for (size_t i = 0; i < e->fluid.size(); ++i) {
             const sph_ctx *c = e->boxes[e->fluid[i]];
@@ -2610,8 +2584,7 @@ static int ens_fluid_plan(sph_ensemble *e)
             }
             itg.push_back(integrate_task(a, b, 0, 10.0, h.tau_x, false, NextHash{}));
             n_itg.push_back((h.np + 255) / 256);
-            if (h.nw > 0) wls.push_back(walls_task(a, b));
-            clk.push_back(ClockTask{b.clock, h.time_dt});
+            end.push_back(StepEndTask{a, step_end(a, b)});
         }
         EnsFluidPhase &P = e->fph[j];
         if ((rc = ens_stage(e, P.hash, hs, n_hs, mem)) || (rc = ens_stage(e, P.rebuild, rb, n_rb, mem)) ||
@@ -2621,11 +2594,9 @@ static int ens_fluid_plan(sph_ensemble *e)
             (rc = ens_stage(e, P.forces[0], frc[0], n_frc[0], mem)) ||
             (rc = ens_stage(e, P.forces[1], frc[1], n_frc[1], mem)) ||
             (rc = ens_stage(e, P.bonds, bnd, n_bnd, mem)) || (rc = ens_stage(e, P.gather, bgt, n_bgt, mem)) ||
-            (rc = ens_stage(e, P.integ, itg, n_itg, mem)) || (rc = ens_array(e, P.walls, wls, mem)) ||
-            (rc = ens_array(e, P.clocks, clk, mem)))
+            (rc = ens_stage(e, P.integ, itg, n_itg, mem)) || (rc = ens_array(e, P.ends, end, mem)))
             return rc;
-        P.nwalls = (uint32_t)wls.size();
-        P.nclocks = (uint32_t)clk.size();
+        P.nends = (uint32_t)end.size();
     }
     // Darcy records (the same for every step)
     std::vector<DarcyTask> all, flux, per2, learned;
@@ -2841,8 +2812,7 @@ static int ens_fluid_step(sph_ensemble *e)
     launch_dm_velocities(s, tc, mc, bc);
     // integration
     launch_integrate_multi(s, (const IntegrateTask *)P.integ.tasks, stage_map(P.integ), P.integ.blocks);
-    launch_walls_multi(s, (const WallsTask *)P.walls, P.nwalls);
-    launch_clock_multi(s, (const ClockTask *)P.clocks, P.nclocks);
+    launch_step_end_multi(s, (const StepEndTask *)P.ends, P.nends);
     (void)hipEventSynchronize(t1);
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, t0, t1);

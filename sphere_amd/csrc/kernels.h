@@ -8,7 +8,7 @@
 #include "resident.h"
 
 // Step counter and simulation time on the device (read by integrate and the
-// wall integration, advanced by k_clock_advance after them), so that a step
+// wall integration, advanced with the walls after them), so that a step
 // replayed from a captured graph sees its own values.
 struct StepClock {
     long long iter;
@@ -70,6 +70,16 @@ struct BondGather {
     const uint8_t *applied;
 };
 
+// What ends a step after integrate (clock == nullptr: nothing): the walls,
+// from the block partials of the wall force, and the clock.
+struct StepEnd {
+    StepClock *clock = nullptr;
+    double4 *w_nx = nullptr, *w_mvfd = nullptr;
+    double *w_acc = nullptr;
+    const double *partial = nullptr;
+    uint32_t nparts = 0;
+};
+
 // The next step's cell hash, formed inside integrate (keys == nullptr: none).
 struct NextHash {
     uint32_t *keys, *vals, *cellc;
@@ -114,19 +124,20 @@ void launch_nl_build(hipStream_t s, const StepArgs &a, const NLArgs &n, const De
 void launch_nl_stats(hipStream_t s, const DemBuffers &b, uint32_t np, uint32_t cap,
                      unsigned long long *out);
 // Contact search (models 2, 3): new overlaps take slots (topology).  near:
-// list mode on a grid searched one cell deep; cur: the step's flag word.
+// list mode on a grid searched one cell deep; cur: the step's flag word; end
+// (list mode): the launch also ends the step before.
 void launch_topology(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool nlist,
-                     bool near, uint32_t cur);
+                     bool near, uint32_t cur, bool end = false);
 // Contact forces, walls and per-particle sums (interact).
 void launch_contact(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool nlist);
 // gather: add the bond forces to force/torque here (else integrate does it)
 void launch_bonds(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool gather);
 void launch_shear_stress(hipStream_t s, const StepArgs &a, const DemBuffers &b);
-void launch_clock_advance(hipStream_t s, StepClock *clock, double dt);
 void launch_integrate(hipStream_t s, const StepArgs &a, const DemBuffers &b,
                       int change_velocity_state, double velocity_factor, double tau_x,
                       bool gather_bonds, const NextHash &nh);
-void launch_integrate_walls(hipStream_t s, const StepArgs &a, const DemBuffers &b);
+// the end of a step: wall integration and the clock's advance
+void launch_step_end(hipStream_t s, const StepArgs &a, const DemBuffers &b);
 void launch_fill_u32(hipStream_t s, uint32_t *p, size_t n, uint32_t v);
 void launch_fill_f64(hipStream_t s, double *p, size_t n, double v);
 void launch_count_contacts(hipStream_t s, const uint64_t *cmask, uint32_t np,
@@ -221,18 +232,9 @@ struct IntegrateTask {
     NextHash nh;
 };
 
-struct WallsTask {
+struct StepEndTask {
     StepArgs a;
-    const StepClock *clock;
-    double4 *w_nx, *w_mvfd;
-    double *w_acc;
-    const double *partial;
-    uint32_t nparts;
-};
-
-struct ClockTask {
-    StepClock *clock;
-    double dt;
+    StepEnd e;
 };
 
 struct HashTask {
@@ -267,7 +269,7 @@ BondTask bond_task(const StepArgs &a, const DemBuffers &b);
 IntegrateTask integrate_task(const StepArgs &a, const DemBuffers &b, int change_velocity_state,
                              double velocity_factor, double tau_x, bool gather_bonds,
                              const NextHash &nh);
-WallsTask walls_task(const StepArgs &a, const DemBuffers &b);
+StepEnd step_end(const StepArgs &a, const DemBuffers &b);
 HashTask hash_task(const StepArgs &a, const NLArgs &n, const DemBuffers &b, uint32_t cur,
                    uint32_t force);
 BondGatherTask bond_gather_task(const DemBuffers &b);
@@ -289,8 +291,8 @@ void launch_integrate_multi(hipStream_t s, const IntegrateTask *t, MultiMap m, u
 void launch_hash_multi(hipStream_t s, const HashTask *t, MultiMap m, uint32_t blocks);
 void launch_bond_gather_multi(hipStream_t s, const BondGatherTask *t, MultiMap m, uint32_t blocks);
 // one block per task
-void launch_walls_multi(hipStream_t s, const WallsTask *t, uint32_t n);
-void launch_clock_multi(hipStream_t s, const ClockTask *t, uint32_t n);
+// the end of a step of n boxes: walls and clock
+void launch_step_end_multi(hipStream_t s, const StepEndTask *t, uint32_t n);
 
 // A max over all the blocks of a launch (the bit pattern of a non-negative
 // double, or NaN above +inf) is kept in RED_LANES words RED_STRIDE words
