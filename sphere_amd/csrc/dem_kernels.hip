@@ -1565,7 +1565,7 @@ __device__ __forceinline__ void topology_lists_body(
     const uint32_t *__restrict__ nl_pos, const uint32_t *__restrict__ cellc,
     const float *__restrict__ nl_gap, const float *__restrict__ nl_gmin,
     const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur,
-    uint32_t bid, uint32_t nblk)
+    uint32_t gpw, uint32_t bid, uint32_t nblk)
 {
     // the list rebuild before it did not finish (its grid barrier timed out)
     if ((*err & ERRF_BARRIER) != 0u) return;
@@ -1576,11 +1576,11 @@ __device__ __forceinline__ void topology_lists_body(
     __shared__ uint8_t s_own[TW * TU], s_k[TW * TU], s_fl[TW * TU];
     const uint32_t lane = threadIdx.x;
     const uint32_t tile = xcd_tile(bid, nblk);
-    const uint32_t pos = tile * TW + lane;
+    const uint32_t pos = tile * gpw + lane;
     const uint32_t np = a.np;
     const Grid &g = a.grid;
     const int NCS = (int)a.nc;
-    const bool valid = pos < np;
+    const bool valid = lane < gpw && pos < np;
     const uint32_t a_orig = valid ? pos : 0u;  // lists are by original index
     // this step's cell from the hash (all ones outside the grid)
     const uint32_t cc = valid ? cellc[pos] : 0xffffffffu;
@@ -1682,7 +1682,7 @@ __device__ __forceinline__ void topology_lists_body(
             bq[u] = 0u;
             sq[u] = 0xffu;
             if (base + t < total) {
-                const size_t li = (size_t)s_k[t] * np + tile * TW + s_own[t];
+                const size_t li = (size_t)s_k[t] * np + tile * gpw + s_own[t];
                 bq[u] = nl[li];
                 sq[u] = nl_slot[li];
             }
@@ -1777,7 +1777,7 @@ __global__ void __launch_bounds__(TW) k_topology_lists(
     uint8_t *__restrict__ slot_cand, const uint32_t *__restrict__ nl_cnt,
     const uint32_t *__restrict__ nl_pos, const uint32_t *__restrict__ cellc,
     const float *__restrict__ nl_gap, const float *__restrict__ nl_gmin,
-    const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur,
+    const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur, uint32_t gpw,
     StepEnd end)
 {
     // The end of the step before: the first block of eight, so that the
@@ -1788,7 +1788,7 @@ __global__ void __launch_bounds__(TW) k_topology_lists(
     }
     topology_lists_body<NEAR>(a, vals, cell_start, cell_end, x, x_s, contacts, cmask, err, nl,
                               nl_slot, slot_cand, nl_cnt, nl_pos, cellc, nl_gap, nl_gmin, nl_disp,
-                              flags_rw, cur, blockIdx.x - 8u, gridDim.x - 8u);
+                              flags_rw, cur, gpw, blockIdx.x - 8u, gridDim.x - 8u);
 }
 
 // Wall contacts of one particle, contactsearch.cuh:420-701: the top wall
@@ -1901,7 +1901,7 @@ __device__ __forceinline__ void forces_body(
     double *__restrict__ delta_t,
     uint8_t *__restrict__ nl_slot, uint8_t *__restrict__ slot_cand,
     const float *__restrict__ nl_gap, float *__restrict__ nl_gmin,
-    const uint32_t *__restrict__ err, uint32_t bid, uint32_t nblk)
+    const uint32_t *__restrict__ err, uint32_t gpw, uint32_t bid, uint32_t nblk)
 {
     // list mode: the list rebuild of this step did not finish
     if (err && (*err & ERRF_BARRIER) != 0u) return;
@@ -1911,9 +1911,9 @@ __device__ __forceinline__ void forces_body(
     __shared__ double s_acc[9][FW];  // the owners' running sums (F, T, es_dot, ev_dot, p)
     const uint32_t lane = threadIdx.x;
     const uint32_t tile = xcd_tile(bid, nblk);
-    const uint32_t pos = tile * FW + lane;
+    const uint32_t pos = tile * gpw + lane;
     const uint32_t np = a.np;
-    const bool valid = pos < np;
+    const bool valid = lane < gpw && pos < np;
     const uint32_t a_orig = valid ? (order ? order[pos] : pos) : 0u;
     const uint64_t mask = valid ? cmask[a_orig] : 0ull;
     const uint32_t n = (uint32_t)__popcll(mask);
@@ -1987,7 +1987,7 @@ __device__ __forceinline__ void forces_body(
                 if (slot_cand) {  // list mode: the list entry loses its slot
                     const uint8_t kk = slot_cand[mempos];
                     if (kk != 0xffu) {
-                        nl_slot[(size_t)kk * np + tile * FW + s_own[lane]] = 0xffu;
+                        nl_slot[(size_t)kk * np + tile * gpw + s_own[lane]] = 0xffu;
                         slot_cand[mempos] = 0xffu;
                         rmk = kk;
                     }
@@ -2053,11 +2053,11 @@ __global__ void __launch_bounds__(FW) k_forces(
     double *__restrict__ delta_t,
     uint8_t *__restrict__ nl_slot, uint8_t *__restrict__ slot_cand,
     const float *__restrict__ nl_gap, float *__restrict__ nl_gmin,
-    const uint32_t *__restrict__ err)
+    const uint32_t *__restrict__ err, uint32_t gpw)
 {
     forces_body<HERTZ>(a, order, x, vel, angvel, force, torque, es_dot_out, ev_dot_out, es, ev,
                        p_out, w_nx, w_mvfd, walls_force_pp, contacts, cmask, delta_t, nl_slot,
-                       slot_cand, nl_gap, nl_gmin, err, blockIdx.x, gridDim.x);
+                       slot_cand, nl_gap, nl_gmin, err, gpw, blockIdx.x, gridDim.x);
 }
 
 // Model 1 (contactLinearViscous + capillary cohesion, no contact history):
@@ -2130,19 +2130,19 @@ void launch_topology(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool
 {
     if (a.prm.contactmodel == 1) return;  // model 1 keeps no contact history
     if (nlist) {
-        const TopoTask t = topology_task(a, b, cur);
-        const uint32_t nw = 8u + (a.np + 63u) / 64u;
+        const TopoTask t = topology_task(a, b, cur, grains_per_wave(a.np));
+        const uint32_t nw = 8u + wave_blocks(a.np, t.gpw);
         const StepEnd e = end ? step_end(a, b) : StepEnd{};
         if (near)
             hipLaunchKernelGGL(k_topology_lists<true>, dim3(nw), dim3(TW), 0, s,
                                t.a, t.vals, t.cell_start, t.cell_end, t.x, t.x_s, t.contacts,
                                t.cmask, t.err, t.nl, t.nl_slot, t.slot_cand, t.nl_cnt, t.nl_pos,
-                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, e);
+                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, t.gpw, e);
         else
             hipLaunchKernelGGL(k_topology_lists<false>, dim3(nw), dim3(TW), 0, s,
                                t.a, t.vals, t.cell_start, t.cell_end, t.x, t.x_s, t.contacts,
                                t.cmask, t.err, t.nl, t.nl_slot, t.slot_cand, t.nl_cnt, t.nl_pos,
-                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, e);
+                               t.cellc, t.nl_gap, t.nl_gmin, t.nl_disp, t.flags, t.cur, t.gpw, e);
     } else
         hipLaunchKernelGGL(k_topology_cells, dim3((a.np + 255) / 256), dim3(256), 0, s, a,
                            b.vals, b.cell_start, b.cell_end, b.x_s, b.contacts, b.cmask,
@@ -2158,18 +2158,18 @@ void launch_contact(hipStream_t s, const StepArgs &a, const DemBuffers &b, bool 
                            b.walls_force_pp, b.errflags);
         return;
     }
-    const ForcesTask t = forces_task(a, b, nlist);
-    const uint32_t nw = (a.np + 63u) / 64u;
+    const ForcesTask t = forces_task(a, b, nlist, grains_per_wave(a.np));
+    const uint32_t nw = wave_blocks(a.np, t.gpw);
     if (a.prm.contactmodel == 3)
         hipLaunchKernelGGL(k_forces<true>, dim3(nw), dim3(FW), 0, s, t.a, t.order, t.x, t.vel,
                            t.angvel, t.force, t.torque, t.es_dot, t.ev_dot, t.es, t.ev, t.p,
                            t.w_nx, t.w_mvfd, t.walls_force_pp, t.contacts, t.cmask, t.delta_t,
-                           t.nl_slot, t.slot_cand, t.nl_gap, t.nl_gmin, t.err);
+                           t.nl_slot, t.slot_cand, t.nl_gap, t.nl_gmin, t.err, t.gpw);
     else
         hipLaunchKernelGGL(k_forces<false>, dim3(nw), dim3(FW), 0, s, t.a, t.order, t.x, t.vel,
                            t.angvel, t.force, t.torque, t.es_dot, t.ev_dot, t.es, t.ev, t.p,
                            t.w_nx, t.w_mvfd, t.walls_force_pp, t.contacts, t.cmask, t.delta_t,
-                           t.nl_slot, t.slot_cand, t.nl_gap, t.nl_gmin, t.err);
+                           t.nl_slot, t.slot_cand, t.nl_gap, t.nl_gmin, t.err, t.gpw);
 }
 
 // ------------------------------------------------------------------
@@ -2719,9 +2719,10 @@ NlBuildTask nl_build_task(const StepArgs &a, const NLArgs &n, const DemBuffers &
     return t;
 }
 
-TopoTask topology_task(const StepArgs &a, const DemBuffers &b, uint32_t cur)
+TopoTask topology_task(const StepArgs &a, const DemBuffers &b, uint32_t cur, uint32_t gpw)
 {
     TopoTask t;
+    t.gpw = gpw;
     t.a = a;
     t.vals = b.vals;
     t.cell_start = b.cell_start;
@@ -2745,9 +2746,10 @@ TopoTask topology_task(const StepArgs &a, const DemBuffers &b, uint32_t cur)
     return t;
 }
 
-ForcesTask forces_task(const StepArgs &a, const DemBuffers &b, bool nlist)
+ForcesTask forces_task(const StepArgs &a, const DemBuffers &b, bool nlist, uint32_t gpw)
 {
     ForcesTask t;
+    t.gpw = gpw;
     t.a = a;
     t.order = nlist ? nullptr : b.vals;  // list mode runs in original order
     t.x = b.x;
@@ -2838,8 +2840,20 @@ StepEnd step_end(const StepArgs &a, const DemBuffers &b)
     return e;
 }
 
-uint32_t topology_blocks(uint32_t np) { return (np + TW - 1) / TW; }
-uint32_t forces_blocks(uint32_t np) { return (np + FW - 1) / FW; }
+// Grains per wave of the search and contact kernels: as many waves as the
+// chip holds of them (256 compute units x 4 SIMDs x 4 waves) before a wave
+// takes more than 16 grains.  A wave's time grows with its grains' contacts, so
+// that a box of few waves waits for its fullest one: 64 grains a wave took
+// 28.3 us per step on 1,000 grains, 30.2 on 10,000 and 64.5 on 87,381 (search
+// 64, contacts 32), the rule 24.0, 27.1 and 61.5.  Fewer than 16 leave most
+// lanes without a contact (8: 27.9 us on 10,000); a full chip is best served
+// by full waves (1,000,000 grains: 390 us, with 32 a wave 412).
+uint32_t grains_per_wave(uint64_t np)
+{
+    const uint64_t g = (np + 4095u) / 4096u;
+    return g < 16u ? 16u : g > 64u ? 64u : (uint32_t)g;
+}
+uint32_t wave_blocks(uint32_t np, uint32_t gpw) { return (np + gpw - 1) / gpw; }
 uint32_t nl_build_blocks(uint32_t np)
 {
     uint32_t nb = (np + 255) / 256;
@@ -2871,7 +2885,7 @@ __global__ void __launch_bounds__(TW) k_topology_multi(const TopoTask *__restric
     const TopoTask &T = t[k];
     topology_lists_body<NEAR>(T.a, T.vals, T.cell_start, T.cell_end, T.x, T.x_s, T.contacts,
                               T.cmask, T.err, T.nl, T.nl_slot, T.slot_cand, T.nl_cnt, T.nl_pos,
-                              T.cellc, T.nl_gap, T.nl_gmin, T.nl_disp, T.flags, T.cur, bid, nblk);
+                              T.cellc, T.nl_gap, T.nl_gmin, T.nl_disp, T.flags, T.cur, T.gpw, bid, nblk);
 }
 
 template <bool HERTZ>
@@ -2882,7 +2896,7 @@ __global__ void __launch_bounds__(FW) k_forces_multi(const ForcesTask *__restric
     const ForcesTask &T = t[k];
     forces_body<HERTZ>(T.a, T.order, T.x, T.vel, T.angvel, T.force, T.torque, T.es_dot, T.ev_dot,
                        T.es, T.ev, T.p, T.w_nx, T.w_mvfd, T.walls_force_pp, T.contacts, T.cmask,
-                       T.delta_t, T.nl_slot, T.slot_cand, T.nl_gap, T.nl_gmin, T.err, bid, nblk);
+                       T.delta_t, T.nl_slot, T.slot_cand, T.nl_gap, T.nl_gmin, T.err, T.gpw, bid, nblk);
 }
 
 __global__ void __launch_bounds__(256) k_bonds_multi(const BondTask *__restrict__ t, MultiMap m)

@@ -2171,6 +2171,13 @@ static std::vector<uint32_t> ens_rebuild_blocks(const sph_ensemble *e, const std
     return nb;
 }
 
+static uint64_t ens_grains(const sph_ensemble *e, const std::vector<int> &ids)
+{
+    uint64_t n = 0;
+    for (int k : ids) n += e->boxes[k]->hs.h.np;
+    return n;
+}
+
 static int ens_plan(sph_ensemble *e)
 {
     ens_drop_plan(e);
@@ -2187,6 +2194,8 @@ static int ens_plan(sph_ensemble *e)
     }
     e->phase = 0;
     const std::vector<uint32_t> rbn = ens_rebuild_blocks(e, e->multi);
+    const uint64_t grains = ens_grains(e, e->multi);
+    const uint32_t gpw = grains_per_wave(grains);
     e->launches_per_step = 0;
     for (int j = 0; j < 2; ++j) {
         std::vector<RebuildTask> rb;
@@ -2218,11 +2227,11 @@ static int ens_plan(sph_ensemble *e)
             nlb.push_back(nl_build_task(a, c->nla, b, cond));
             n_nlb.push_back((h.np + 255) / 256);
             const int near = c->nla.range == 1 ? 1 : 0;
-            topo[near].push_back(topology_task(a, b, cur));
-            n_topo[near].push_back(topology_blocks(h.np));
+            topo[near].push_back(topology_task(a, b, cur, gpw));
+            n_topo[near].push_back(wave_blocks(h.np, gpw));
             const int hz = h.contactmodel == 3 ? 1 : 0;
-            frc[hz].push_back(forces_task(a, b, true));
-            n_frc[hz].push_back(forces_blocks(h.np));
+            frc[hz].push_back(forces_task(a, b, true, gpw));
+            n_frc[hz].push_back(wave_blocks(h.np, gpw));
             if (h.nb0 > 0) {
                 bnd.push_back(bond_task(a, b));
                 n_bnd.push_back((h.nb0 + 255) / 256);
@@ -2534,6 +2543,8 @@ static int ens_fluid_plan(sph_ensemble *e)
     e->fl_maxiter = e->boxes[e->fluid[0]]->hs.h.maxiter;
     e->fl_phase = 0;
     const std::vector<uint32_t> rbn = ens_rebuild_blocks(e, e->fluid);
+    const uint64_t grains = ens_grains(e, e->fluid);
+    const uint32_t gpw = grains_per_wave(grains);
     int rc;
     for (int j = 0; j < 2; ++j) {
         std::vector<HashTask> hs;
@@ -2569,11 +2580,11 @@ static int ens_fluid_plan(sph_ensemble *e)
             nlb.push_back(nl_build_task(a, c->nla, b, cond));
             n_nlb.push_back((h.np + 255) / 256);
             const int near = c->nla.range == 1 ? 1 : 0;
-            topo[near].push_back(topology_task(a, b, cur));
-            n_topo[near].push_back(topology_blocks(h.np));
+            topo[near].push_back(topology_task(a, b, cur, gpw));
+            n_topo[near].push_back(wave_blocks(h.np, gpw));
             const int hz = h.contactmodel == 3 ? 1 : 0;
-            frc[hz].push_back(forces_task(a, b, true));
-            n_frc[hz].push_back(forces_blocks(h.np));
+            frc[hz].push_back(forces_task(a, b, true, gpw));
+            n_frc[hz].push_back(wave_blocks(h.np, gpw));
             if (h.nb0 > 0) {
                 bnd.push_back(bond_task(a, b));
                 n_bnd.push_back((h.nb0 + 255) / 256);

@@ -187,6 +187,7 @@ struct TopoTask {
     const float *nl_gap, *nl_gmin, *nl_disp;
     uint32_t *flags;
     uint32_t cur;
+    uint32_t gpw;  // grains per wave
 };
 
 struct ForcesTask {
@@ -205,6 +206,7 @@ struct ForcesTask {
     const float *nl_gap;
     float *nl_gmin;
     const uint32_t *err;
+    uint32_t gpw;  // grains per wave
 };
 
 struct BondTask {
@@ -263,8 +265,8 @@ RebuildTask rebuild_task(const StepArgs &a, const DemBuffers &b, uint32_t ncells
                          const uint32_t *cond, uint32_t spin_limit);
 NlBuildTask nl_build_task(const StepArgs &a, const NLArgs &n, const DemBuffers &b,
                           const uint32_t *cond);
-TopoTask topology_task(const StepArgs &a, const DemBuffers &b, uint32_t cur);
-ForcesTask forces_task(const StepArgs &a, const DemBuffers &b, bool nlist);
+TopoTask topology_task(const StepArgs &a, const DemBuffers &b, uint32_t cur, uint32_t gpw);
+ForcesTask forces_task(const StepArgs &a, const DemBuffers &b, bool nlist, uint32_t gpw);
 BondTask bond_task(const StepArgs &a, const DemBuffers &b);
 IntegrateTask integrate_task(const StepArgs &a, const DemBuffers &b, int change_velocity_state,
                              double velocity_factor, double tau_x, bool gather_bonds,
@@ -274,8 +276,10 @@ HashTask hash_task(const StepArgs &a, const NLArgs &n, const DemBuffers &b, uint
                    uint32_t force);
 BondGatherTask bond_gather_task(const DemBuffers &b);
 // Blocks a box needs in each multi-box stage.
-uint32_t topology_blocks(uint32_t np);
-uint32_t forces_blocks(uint32_t np);
+// grains of one wave in the search and contact kernels, for a launch over np
+// grains, and the waves that np grains then take
+uint32_t grains_per_wave(uint64_t np);
+uint32_t wave_blocks(uint32_t np, uint32_t gpw);
 uint32_t nl_build_blocks(uint32_t np);
 // Multi-box launches of `blocks` blocks (the last start plus its count,
 // rounded up) over device task arrays; near/hertz pick the kernel variant
