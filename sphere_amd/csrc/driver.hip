@@ -70,6 +70,7 @@ struct sph_ctx {
     uint32_t nl_parity = 0;
     uint32_t nl_force = 1;
     bool hash_ready = false;  // the last integrate formed this step's hash
+    bool hash_aside = false;  // ... in keys_tmp and vals_tmp
     // time loop host variables, src/device.cu:913-1036
     long iter = 0;
     double filetimeclock = 0.0;
@@ -595,7 +596,7 @@ static int upload(sph_ctx *ctx)
     }
     ctx->nl_parity = 0;
     ctx->nl_force = 1;
-    ctx->hash_ready = false;
+    ctx->hash_ready = ctx->hash_aside = false;
 #undef AL
     ctx->iter = 0;
     ctx->gen++;
@@ -1279,22 +1280,30 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
         const StepArgs a = step_args(ctx);
         if (ctx->nl_on) {
             // Lists are rebuilt (sort, reorder, list build) only on steps
-            // whose device-side flag is set; the Darcy solve reads the
-            // sorted arrays, so a fluid run rebuilds every step.
+            // whose device-side flag is set.  The fluids read the sorted
+            // arrays, so with a fluid the sort and reorder run every step
+            // (as launches of their own, which full grids make faster than
+            // the rebuild kernel's barriers), the list build on flagged steps.
+            const bool fluid = h.fluid || ctx->ns;
             const uint32_t cur = ctx->nl_parity;
             const uint32_t *cond = ctx->db.nl_flags + cur;
-            const uint32_t force = ctx->nl_force || h.fluid || ctx->ns ? 1u : 0u;
-            if (force || !ctx->hash_ready) {  // else the last integrate formed the hash
+            const uint32_t force = ctx->nl_force || !ctx->hash_ready ? 1u : 0u;
+            if (force) {  // else the last integrate formed the hash
                 ProfScope ps(ctx, SPH_K_HASH);
                 launch_hash_nl(s, a, ctx->nla, ctx->db, cur, force);
+            } else if (ctx->hash_aside) {
+                std::swap(ctx->db.keys, ctx->db.keys_tmp);
+                std::swap(ctx->db.vals, ctx->db.vals_tmp);
             }
-            if (ctx->rb_blocks) {
+            ctx->hash_aside = false;
+            if (ctx->rb_blocks && !fluid) {
                 ProfScope ps(ctx, SPH_K_NLIST);
                 launch_rebuild(s, a, ctx->nla, ctx->db, ctx->ncells, ctx->key_bits,
                                ctx->rb_blocks, cond, ctx->rb_spin);
             } else {
-                { ProfScope ps(ctx, SPH_K_SORT); launch_sort(s, a.np, ctx->key_bits, ctx->db, cond); }
-                { ProfScope ps(ctx, SPH_K_REORDER); launch_reorder(s, a, ctx->db, ctx->ncells, cond); }
+                const uint32_t *sort = fluid ? nullptr : cond;
+                { ProfScope ps(ctx, SPH_K_SORT); launch_sort(s, a.np, ctx->key_bits, ctx->db, sort); }
+                { ProfScope ps(ctx, SPH_K_REORDER); launch_reorder(s, a, ctx->db, ctx->ncells, sort); }
                 { ProfScope ps(ctx, SPH_K_NLIST); launch_nl_build(s, a, ctx->nla, ctx->db, cond); }
             }
             { ProfScope ps(ctx, SPH_K_TOPOLOGY);
@@ -1345,13 +1354,14 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
             change_velocity_state = -1;
             ctx->velocity_state = 1;
         }
-        // Without fluid the next step's cell hash is formed by integrate (list
-        // mode); the fluid step rebuilds and hashes every step.
+        // In list mode the next step's cell hash is formed by integrate; with
+        // a fluid beside the sorted keys, which stay readable after the step.
         NextHash nh{};
-        const bool fuse_hash = ctx->nl_on && !h.fluid;
+        const bool fuse_hash = ctx->nl_on;
         if (fuse_hash) {
-            nh.keys = ctx->db.keys;
-            nh.vals = ctx->db.vals;
+            ctx->hash_aside = h.fluid || ctx->ns;
+            nh.keys = ctx->hash_aside ? ctx->db.keys_tmp : ctx->db.keys;
+            nh.vals = ctx->hash_aside ? ctx->db.vals_tmp : ctx->db.vals;
             nh.cellc = ctx->db.cellc;
             nh.x_ref = ctx->db.x_ref;
             nh.disp = ctx->db.nl_disp;
@@ -1420,6 +1430,7 @@ sph_ctx *sph_create(int device)
 int sph_ns_attach(sph_ns *ns, sph_ctx *ctx)
 {
     if (!ctx) return fail(ctx, SPH_ERR_ARG, "null context");
+    ctx->hash_ready = ctx->hash_aside = false;  // the next step hashes anew
     if (!ns) {
         if (ctx->ns) ns_set_attached(ctx->ns, 0);
         ctx->ns = nullptr;
@@ -2859,7 +2870,7 @@ static int ens_fluid_step(sph_ensemble *e)
                     c->iter, c->iter * c->hs.h.time_dt, maxiter, c->hs.h.tolerance);
         }
         ens_host_advance(c);
-        c->hash_ready = false;  // a fluid step hashes every step
+        c->hash_ready = c->hash_aside = false;  // a fluid step of an ensemble hashes every step
     }
     e->fl_phase ^= 1u;
     e->fluid_steps++;
@@ -2970,7 +2981,7 @@ int sph_ensemble_step(sph_ensemble *e, int nsteps)
         for (int k : e->multi) {
             sph_ctx *c = e->boxes[k];
             if (c->nl_force || !c->hash_ready) {
-                launch_hash_nl(e->stream, step_args(c), c->nla, c->db, c->nl_parity, c->nl_force ? 1u : 0u);
+                launch_hash_nl(e->stream, step_args(c), c->nla, c->db, c->nl_parity, 1u);
                 hashed = true;
             }
         }
