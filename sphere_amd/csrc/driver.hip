@@ -792,7 +792,7 @@ static int darcy_correct(sph_ctx *ctx, const DarcyArgs &da, double *pc)
     const DarcyBuffers &d = ctx->dd;
     launch_darcy_residual_max(s, da, d, pc, false);
     launch_darcy_net_input(s, da, d, pc, nullptr, false, net_input_bf16(ctx->net));
-    const int rc = net_forward_packed(ctx->net, ctx->net_params, nullptr, ctx->net_out, s);
+    const int rc = net_forward_packed(ctx->net, ctx->net_params, ctx->net_out, s);
     if (rc) return fail(ctx, rc, sph_net_last_error());
     launch_darcy_net_apply(s, da, d, pc, ctx->net_out);
     return SPH_OK;

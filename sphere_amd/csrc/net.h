@@ -3,10 +3,11 @@
 #include <hip/hip_runtime.h>
 #include "../../include/sphere_hip.h"
 
-// BF16 copies of the FP32 parameters for the passes that follow
-void net_pack(sph_net *n, const float *params, hipStream_t s);
-// forward pass (input [V][3] -> output [V]) with the last packed weights
-int net_forward_packed(sph_net *n, const float *params, const float *input, float *output, hipStream_t s);
+// BF16 copies of the FP32 parameters for the passes that follow, and of the
+// input ([V][3] FP32; null: the caller fills the rows of net_input_bf16)
+void net_pack(sph_net *n, const float *params, hipStream_t s, const float *input = nullptr);
+// forward pass (output [V]) of the input rows with the last packed weights
+int net_forward_packed(sph_net *n, const float *params, float *output, hipStream_t s);
 uint16_t *net_input_bf16(sph_net *n);
 
 // The forward passes of several networks (the boxes of an ensemble, each

@@ -82,7 +82,6 @@ struct sph_net {
     // gradients (FP32) and the BF16 operand of the weight gradient
     float *d_h0, *d_y0, *d_a1, *d_y1, *d_a2, *d_y2, *d_a3, *d_x3, *d_p2, *d_p1, *d_p0;
     uint16_t *dz;
-    float *gw;
 };
 
 static bool net_alloc(sph_net *n, void **p, size_t bytes)
@@ -174,7 +173,6 @@ sph_net *sph_net_create(int device, uint32_t nx, uint32_t ny, uint32_t nz, uint3
     A32(&n->d_p2, (size_t)V[3] * 48); A32(&n->d_p1, (size_t)V[2] * 32);
     A32(&n->d_p0, (size_t)V[1] * 16);
     A16(&n->dz, (size_t)V[0] * 16);
-    A32(&n->gw, 27ull * 64 * 64);
     (void)hipSetDevice(prev);
     if (!ok) {
         g_net_error = "device allocation failed";
@@ -187,28 +185,32 @@ sph_net *sph_net_create(int device, uint32_t nx, uint32_t ny, uint32_t nz, uint3
 }  // extern "C"
 
 // BF16 operand copies of the FP32 parameters (forward and adjoint layouts)
-void net_pack(sph_net *n, const float *params, hipStream_t s)
+// and, with input != null, of the network's input
+void net_pack(sph_net *n, const float *params, hipStream_t s, const float *input)
 {
+    PackLayers p{};
     for (int l = 0; l < 9; ++l) {
         const LayerSpec &L = kLayers[l];
         if (L.taps != 27) continue;
-        launch_pack_weights(s, params + n->woff[l], L.cin, L.cout, n->wf[l], pad_in(L.cin), pad_out(L.cout),
-                            n->wt[l], pad_in(L.cout), pad_out(L.cin));
+        p.layer[p.n++] = PackLayer{params + n->woff[l], L.cin, L.cout, n->wf[l], pad_in(L.cin), pad_out(L.cout),
+                                   n->wt[l], pad_in(L.cout), pad_out(L.cin), 0u};
     }
+    p.in = input;
+    p.in4 = n->in4;
+    p.V = n->V[0];
+    launch_pack_weights(s, p);
 }
 
-// the network's BF16 input rows (V x 4), which a caller may fill itself and
-// then pass a null input to net_forward_packed
+// the network's BF16 input rows (V x 4), filled by net_pack or by the caller
 uint16_t *net_input_bf16(sph_net *n) { return n->in4; }
 
-// forward pass with the weights of the last net_pack
-int net_forward_packed(sph_net *n, const float *params, const float *input, float *output, hipStream_t s)
+// forward pass of the input rows with the weights of the last net_pack
+int net_forward_packed(sph_net *n, const float *params, float *output, hipStream_t s)
 {
     const NetGeom *g = n->g;
     const float *b[9];
     for (int l = 0; l < 9; ++l) b[l] = params + n->boff[l];
     int rc = 0;
-    if (input) launch_to_bf16_pad(s, n->V[0], input, 3, 4, n->in4);  // else in4 is filled
     rc |= launch_conv_fwd(s, g[0], n->in4, 4, n->wf[0], 16, b[0], 16, n->x0, NET_OUT_BF16_RELU);
     launch_pool_fwd(s, g[1], n->x0, 16, n->p0);
     rc |= launch_conv_fwd(s, g[1], n->p0, 16, n->wf[1], 32, b[1], 32, n->x1, NET_OUT_BF16_RELU);
@@ -396,8 +398,8 @@ int sph_net_forward(sph_net *n, const float *params, const float *input, float *
         g_net_error = "null argument";
         return SPH_ERR_ARG;
     }
-    net_pack(n, params, (hipStream_t)stream);
-    return net_forward_packed(n, params, input, output, (hipStream_t)stream);
+    net_pack(n, params, (hipStream_t)stream, input);
+    return net_forward_packed(n, params, output, (hipStream_t)stream);
 }
 
 // Backward pass of the last forward: grad_output[V0] FP32 (dLoss/dout);
@@ -414,55 +416,46 @@ int sph_net_backward(sph_net *n, const float *params, const float *grad_output, 
     const NetGeom *g = n->g;
     const uint32_t *V = n->V;
     int rc = 0;
-    // weight and bias gradient of layer l from input x (cin_x channels) and
-    // the BF16 output gradient in n->dz (cdz channels)
-    auto wgrad = [&](int l, const uint16_t *x, int cin_x, int cdz, int level) {
+    // layer l's output gradient dy masked by its ReLU output y into n->dz
+    // (BF16), its bias gradient, and its weight gradient from input x (cin_x
+    // channels)
+    auto wgrad = [&](int l, const float *dy, const uint16_t *y, const uint16_t *x, int cin_x, int level) {
         const LayerSpec &L = kLayers[l];
-        launch_fill_f32(s, n->gw, 27ull * cdz * cin_x, 0.f);
-        rc |= launch_conv_wgrad(s, g[level], x, cin_x, n->dz, cdz, n->gw);
-        launch_unpack_wgrad(s, n->gw, L.cin, cin_x, L.cout, cdz, grad_params + n->woff[l]);
-        launch_bias_grad(s, V[level], n->dz, cdz, L.cout, grad_params + n->boff[l]);
+        launch_relu_mask(s, V[level], dy, y, L.cout, n->dz, grad_params + n->boff[l]);
+        rc |= launch_conv_wgrad(s, g[level], x, cin_x, n->dz, L.cout, grad_params + n->woff[l], L.cin);
     };
     // c8: out = w8 . h0 + b8 (weights and bias contiguous)
     launch_proj_bwd(s, V[0], grad_output, n->h0, params + n->woff[8], n->d_h0, grad_params + n->woff[8]);
     // c7: h0 = relu(conv(y0))
-    launch_relu_mask(s, V[0], n->d_h0, n->h0, 16, 16, n->dz);
-    wgrad(7, n->y0, 16, 16, 0);
+    wgrad(7, n->d_h0, n->h0, n->y0, 16, 0);
     rc |= launch_conv_fwd(s, g[0], n->dz, 16, n->wt[7], 16, nullptr, 16, n->d_y0, NET_OUT_F32);
     // y0 = up(a1) + x0: d_y0 is also the gradient of x0 (accumulated below)
     launch_up_bwd(s, g[1], n->d_y0, 16, n->d_a1);
     // c6: a1 = relu(conv(y1))
-    launch_relu_mask(s, V[1], n->d_a1, n->a1, 16, 16, n->dz);
-    wgrad(6, n->y1, 32, 16, 1);
+    wgrad(6, n->d_a1, n->a1, n->y1, 32, 1);
     rc |= launch_conv_fwd(s, g[1], n->dz, 16, n->wt[6], 32, nullptr, 32, n->d_y1, NET_OUT_F32);
     launch_up_bwd(s, g[2], n->d_y1, 32, n->d_a2);
     // c5: a2 = relu(conv(y2))
-    launch_relu_mask(s, V[2], n->d_a2, n->a2, 32, 32, n->dz);
-    wgrad(5, n->y2, 48, 32, 2);
+    wgrad(5, n->d_a2, n->a2, n->y2, 48, 2);
     rc |= launch_conv_fwd(s, g[2], n->dz, 32, n->wt[5], 48, nullptr, 48, n->d_y2, NET_OUT_F32);
     launch_up_bwd(s, g[3], n->d_y2, 48, n->d_a3);
     // c4: a3 = relu(conv(x3))
-    launch_relu_mask(s, V[3], n->d_a3, n->a3, 48, 48, n->dz);
-    wgrad(4, n->x3, 64, 48, 3);
+    wgrad(4, n->d_a3, n->a3, n->x3, 64, 3);
     rc |= launch_conv_fwd(s, g[3], n->dz, 48, n->wt[4], 64, nullptr, 64, n->d_x3, NET_OUT_F32);
     // c3: x3 = relu(conv(p2))
-    launch_relu_mask(s, V[3], n->d_x3, n->x3, 64, 64, n->dz);
-    wgrad(3, n->p2, 48, 64, 3);
+    wgrad(3, n->d_x3, n->x3, n->p2, 48, 3);
     rc |= launch_conv_fwd(s, g[3], n->dz, 64, n->wt[3], 48, nullptr, 48, n->d_p2, NET_OUT_F32);
     launch_pool_bwd(s, g[2], n->d_p2, 48, n->d_y2);  // x2's gradient: skip + pool paths
     // c2: x2 = relu(conv(p1))
-    launch_relu_mask(s, V[2], n->d_y2, n->x2, 48, 48, n->dz);
-    wgrad(2, n->p1, 32, 48, 2);
+    wgrad(2, n->d_y2, n->x2, n->p1, 32, 2);
     rc |= launch_conv_fwd(s, g[2], n->dz, 48, n->wt[2], 32, nullptr, 32, n->d_p1, NET_OUT_F32);
     launch_pool_bwd(s, g[1], n->d_p1, 32, n->d_y1);
     // c1: x1 = relu(conv(p0))
-    launch_relu_mask(s, V[1], n->d_y1, n->x1, 32, 32, n->dz);
-    wgrad(1, n->p0, 16, 32, 1);
+    wgrad(1, n->d_y1, n->x1, n->p0, 16, 1);
     rc |= launch_conv_fwd(s, g[1], n->dz, 32, n->wt[1], 16, nullptr, 16, n->d_p0, NET_OUT_F32);
     launch_pool_bwd(s, g[0], n->d_p0, 16, n->d_y0);
     // c0: x0 = relu(conv(in))
-    launch_relu_mask(s, V[0], n->d_y0, n->x0, 16, 16, n->dz);
-    wgrad(0, n->in4, 4, 16, 0);
+    wgrad(0, n->d_y0, n->x0, n->in4, 4, 0);
     if (rc) {
         g_net_error = "unsupported layer shape";
         return SPH_ERR_VALUE;
@@ -472,6 +465,14 @@ int sph_net_backward(sph_net *n, const float *params, const float *grad_output, 
         return SPH_ERR_HIP;
     }
     return SPH_OK;
+}
+
+static void pack_one(hipStream_t s, const float *w, int cin, int cout, uint16_t *wf, int cpad, int opad)
+{
+    PackLayers p{};
+    p.n = 1;
+    p.layer[0] = PackLayer{w, cin, cout, wf, cpad, opad, nullptr, 0, 0, 0u};
+    launch_pack_weights(s, p);
 }
 
 // One 3x3x3 convolution as the network runs it, for tests: in[V][cin]
@@ -502,7 +503,7 @@ int sph_net_conv3d(const float *in, int cin, const float *w, const float *b, int
         return SPH_ERR_HIP;
     }
     launch_to_bf16_pad(s, V, in, cin, cpad, inb);
-    launch_pack_weights(s, w, cin, cout, wf, cpad, opad, nullptr, 0, 0);
+    pack_one(s, w, cin, cout, wf, cpad, opad);
     int rc = launch_conv_fwd(s, g, inb, cpad, wf, opad, b, cout, out, NET_OUT_F32);
     (void)hipStreamSynchronize(s);
     (void)hipFree(inb);
@@ -546,7 +547,7 @@ int sph_net_conv3d_noalloc(const float *in, int cin, const float *w, const float
     // the staging kernels write every element they reserve (padding as
     // zeros), so nothing in the scratch needs clearing between calls
     launch_to_bf16_pad(s, (uint32_t)V64, in, cin, cpad, inb);
-    launch_pack_weights(s, w, cin, cout, wf, cpad, opad, nullptr, 0, 0);
+    pack_one(s, w, cin, cout, wf, cpad, opad);
     if (launch_conv_fwd(s, g, inb, cpad, wf, opad, b, cout, out, NET_OUT_F32)) {
         g_net_error = "unsupported shape";
         return SPH_ERR_VALUE;

@@ -42,22 +42,35 @@ int launch_conv_fwd(hipStream_t s, const NetGeom &g, const uint16_t *in, int cin
                     const uint16_t *skip = nullptr, uint16_t *yfine = nullptr);
 void launch_proj_bwd(hipStream_t s, uint32_t V, const float *dout, const uint16_t *h, const float *w, float *dh,
                      float *g);
-// dw[27][cout][cin] += sum_v dz[v][co] x[v + tap][ci]; x[V][cin] (cin 4 or
-// a multiple of 16), dz[V][cout]
+// dw[27][cout][cin_real] += sum_v dz[v][co] x[v + tap][ci]; x[V][cin] (cin 4
+// or a multiple of 16, of which the first cin_real count), dz[V][cout] (cout a
+// multiple of 16)
 int launch_conv_wgrad(hipStream_t s, const NetGeom &g, const uint16_t *x, int cin, const uint16_t *dz,
-                      int cout, float *dw);
-void launch_bias_grad(hipStream_t s, uint32_t V, const uint16_t *dz, int c_stride, int c_real, float *db);
+                      int cout, float *dw, int cin_real);
 void launch_pool_fwd(hipStream_t s, const NetGeom &gc, const uint16_t *in, int c, uint16_t *out);
 void launch_pool_bwd(hipStream_t s, const NetGeom &gf, const float *dcoarse, int c, float *dfine);
 void launch_up_bwd(hipStream_t s, const NetGeom &gc, const float *dfine, int c, float *dcoarse);
-void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t *y, int c, int cpad,
-                      uint16_t *dz);
+// dz = bf16(dy where y > 0), db += sum_v dz; c a multiple of 4 up to 64
+void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t *y, int c, uint16_t *dz,
+                      float *db);
 void launch_to_bf16_pad(hipStream_t s, uint32_t V, const float *in, int c, int cpad, uint16_t *out);
-void launch_pack_weights(hipStream_t s, const float *w, int cin, int cout, uint16_t *wf, int cin_pad,
-                         int cout_pad, uint16_t *wt, int tin_pad, int tout_pad);
-void launch_unpack_wgrad(hipStream_t s, const float *gw, int cin, int cin_pad, int cout, int cout_pad,
-                         float *g);
-void launch_fill_f32(hipStream_t s, float *p, size_t n, float v);
+struct PackLayer {
+    const float *w;
+    int cin, cout;
+    uint16_t *wf;
+    int cin_pad, cout_pad;
+    uint16_t *wt;  // or null
+    int tin_pad, tout_pad;
+    uint32_t blocks;  // set by the launcher: blocks up to this layer's end
+};
+struct PackLayers {
+    PackLayer layer[8];
+    int n;
+    const float *in;  // V rows of 3 to convert, or null
+    uint16_t *in4;
+    uint32_t V;
+};
+void launch_pack_weights(hipStream_t s, PackLayers &p);
 
 // Multi-box launches of the forward pass (ensembles): one task record per
 // box and layer, the arguments of launch_conv_fwd / launch_pool_fwd.  The

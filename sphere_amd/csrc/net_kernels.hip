@@ -675,125 +675,151 @@ void launch_proj_bwd(hipStream_t s, uint32_t V, const float *dout, const uint16_
 // ---------------------------------------------------------------------------
 // Weight gradient dW[tap][co][ci] += sum_v dz[v][co] x[v + tap][ci] as
 // MFMA tiles with M = 16 output channels, N = 16 input channels (CIN4: four
-// taps of 4 channels) and K = 16 voxels per step.  One wave sums a chunk of
-// WG_VOX voxels for one tap (CIN4: one group of four taps) and one (co, ci)
-// tile, then adds its 16x16 partial to dW with FP32 atomics.
+// taps of 4 channels) and K = 32 voxels per step.
+//
+// The contraction runs over voxels, so both operands are wanted eight voxels
+// per lane while the activations are channels-last.  A block therefore stages
+// a tile of 16 x 4 x 4 voxels transposed in LDS: dz as [channel][voxel], and x
+// with its halo as three copies [channel][row][x], one for each x offset of a
+// tap, so that every operand is one aligned 16-byte read.  The channel
+// strides (528 and 1168 bytes) spread the 16 channels of a read over all 64
+// banks.  Each of the four waves holds the 16 x 16 sums of seven taps (CIN4:
+// two groups of four) over all of the block's tiles and adds them to dW with
+// FP32 atomics at the end.  On the 48 x 48 x 96 grid a layer takes
+// 9 to 27 us, the input layer 33, where one 2-byte load and one voxel division
+// per operand element took 76 us on average and 107.
 // ---------------------------------------------------------------------------
-#define WG_VOX 1024
+#define WT_X 16
+#define WT_Y 4
+#define WT_Z 4
+#define WT_ROWS (WT_Y * WT_Z)                 // x rows of the tile
+#define WT_HROWS ((WT_Y + 2) * (WT_Z + 2))    // x rows with the halo
+#define WT_DZ_CH (WT_ROWS * WT_X + 8)         // channel strides, elements
+#define WT_X_CH (WT_HROWS * WT_X + 8)
+// Blocks a launch aims at: two per compute unit, and fewer for the input
+// layer, whose 1,296 sums every block adds to (432 blocks took 60 us, 124
+// blocks 33; the 16 to 16 channel layer with 6,912 sums 27 us with
+// 432 blocks, 31 with 216).
+#define WT_BLOCKS 512u
+#define WT_BLOCKS_IN 128u
 
 template <bool CIN4>
 __global__ void __launch_bounds__(256) k_conv_wgrad(NetGeom g, const uint16_t *__restrict__ x, int cin,
                                                     const uint16_t *__restrict__ dz, int cout,
-                                                    float *__restrict__ dw, uint32_t ntaps,
-                                                    uint32_t nco, uint32_t nci, uint32_t nchunk)
+                                                    float *__restrict__ dw, int cin_real, uint32_t ntx,
+                                                    uint32_t nty, uint32_t ntiles, uint32_t per,
+                                                    uint32_t nci, uint32_t nchunk)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t job = blockIdx.x * 4u + (threadIdx.x >> 6);
-    const uint32_t total = ntaps * nco * nci * nchunk;
-    if (job >= total) return;
+    constexpr int XC = CIN4 ? 4 : 16;   // staged input channels
+    constexpr int NT = CIN4 ? 2 : 7;    // tap groups of a wave
+    __shared__ __align__(16) uint16_t s_dz[16 * WT_DZ_CH];
+    __shared__ __align__(16) uint16_t s_x[3 * XC * WT_X_CH];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint32_t job = blockIdx.x;
     const uint32_t chunk = job % nchunk;
     job /= nchunk;
-    const uint32_t cit = job % nci;
-    job /= nci;
-    const uint32_t cot = job % nco;
-    const uint32_t tg = job / nco;  // tap (CIN4: group of four taps)
+    const uint32_t cit = job % nci, cot = job / nci;
     const uint32_t m = lane & 15u, grp = lane >> 4;
-    const uint32_t V = g.nx * g.ny * g.nz;
-    // the lane's B column: input channel (CIN4: tap of the group, channel)
-    int tap, ci;
-    if (CIN4) {
-        tap = (int)(tg * 4u + (m >> 2));
-        ci = (int)(m & 3u);
-    } else {
-        tap = (int)tg;
-        ci = (int)(cit * 16u + m);
-    }
-    const bool tok = tap < 27;
-    const int dzz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dxx = tap % 3 - 1;
-    const int co = (int)(cot * 16u + m);
-    const bool cok = co < cout;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t vb = chunk * WG_VOX;
-    const uint32_t ve = vb + WG_VOX < V ? vb + WG_VOX : V;
-    for (uint32_t k0 = vb; k0 < ve; k0 += 16u) {
-        bf16x4 a, b;
+    f32x4 acc[NT];
+    int xoff[NT];  // this lane's B rows of each tap group: copy, channel, tap's y and z
+    bool tok[NT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t v = k0 + 4u * grp + (uint32_t)i;
-            short av = 0, bv = 0;
-            if (v < ve) {
-                if (cok) av = (short)dz[(size_t)v * cout + co];
-                if (tok) {
-                    int vx, vy, vz;
-                    vox_xyz(g, v, vx, vy, vz);
-                    int xx = vx + dxx, yy = vy + dyy;
-                    const int zz = vz + dzz;
-                    if (nb_in(g, xx, yy, zz))
-                        bv = (short)x[(size_t)((zz * (int)g.ny + yy) * (int)g.nx + xx) * cin + ci];
+    for (int t = 0; t < NT; ++t) {
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int q = (int)wave * NT + t;
+        const int tap = CIN4 ? q * 4 + (int)(m >> 2) : q;
+        const int ci = CIN4 ? (int)(m & 3u) : (int)m;
+        tok[t] = tap < 27;
+        const int tt = tok[t] ? tap : 13;
+        xoff[t] = ((tt % 3) * XC + ci) * WT_X_CH + ((tt / 9) * (WT_Y + 2) + (tt / 3) % 3) * WT_X;
+    }
+    const uint32_t t1 = (chunk + 1u) * per < ntiles ? (chunk + 1u) * per : ntiles;
+    for (uint32_t tile = chunk * per; tile < t1; ++tile) {
+        const int bx = (int)(tile % ntx) * WT_X, by = (int)((tile / ntx) % nty) * WT_Y;
+        const int bz = (int)(tile / (ntx * nty)) * WT_Z;
+        __syncthreads();
+        // dz: 256 voxels x 16 channels, 8 channels per item
+        for (uint32_t i = tid; i < 2u * WT_ROWS * WT_X; i += 256u) {
+            const uint32_t half = i & 1u, v = i >> 1;
+            const int vx = bx + (int)(v % WT_X), vy = by + (int)((v / WT_X) % WT_Y);
+            const int vz = bz + (int)(v / (WT_X * WT_Y));
+            s16x8 q = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (vx < (int)g.nx && vy < (int)g.ny && vz < (int)g.nz)
+                q = *(const s16x8 *)(dz + (size_t)((vz * (int)g.ny + vy) * (int)g.nx + vx) * cout + cot * 16u +
+                                     half * 8u);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) s_dz[(half * 8u + c) * WT_DZ_CH + v] = (uint16_t)q[c];
+        }
+        // x with its halo: 18 x 6 x 6 voxels
+        constexpr uint32_t HV = (WT_X + 2) * WT_HROWS, PARTS = CIN4 ? 1u : 2u;
+        for (uint32_t i = tid; i < HV * PARTS; i += 256u) {
+            const uint32_t half = CIN4 ? 0u : i & 1u, v = CIN4 ? i : i >> 1;
+            const uint32_t hx = v % (WT_X + 2), row = v / (WT_X + 2);
+            int vx = bx + (int)hx - 1, vy = by + (int)(row % (WT_Y + 2)) - 1;
+            const int vz = bz + (int)(row / (WT_Y + 2)) - 1;
+            s16x8 q = {0, 0, 0, 0, 0, 0, 0, 0};
+            // a tile may reach past the grid: only true neighbours of its voxels
+            if (vx <= (int)g.nx && vy <= (int)g.ny && nb_in(g, vx, vy, vz)) {
+                const uint16_t *p = x + (size_t)((vz * (int)g.ny + vy) * (int)g.nx + vx) * cin;
+                if (CIN4) {
+                    const bf16x4 h = *(const bf16x4 *)p;
+                    q[0] = h[0], q[1] = h[1], q[2] = h[2], q[3] = h[3];
+                } else {
+                    q = *(const s16x8 *)(p + cit * 16u + half * 8u);
                 }
             }
-            a[i] = av;
-            b[i] = bv;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {  // copy d holds x[t + d - 1] at t
+                const int t = (int)hx - d;
+                if (t < 0 || t >= WT_X) continue;
+#pragma unroll
+                for (int c = 0; c < (CIN4 ? 4 : 8); ++c)
+                    s_x[((uint32_t)(d * XC) + half * 8u + c) * WT_X_CH + row * WT_X + t] = (uint16_t)q[c];
+            }
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t ks = 0; ks < WT_ROWS / 2u; ++ks) {
+            const uint32_t r = 2u * ks + (grp >> 1), x8 = 8u * (grp & 1u);
+            const s16x8 a = *(const s16x8 *)(s_dz + m * WT_DZ_CH + r * WT_X + x8);
+            const uint32_t rx = ((r / WT_Y) * (WT_Y + 2) + r % WT_Y) * WT_X + x8;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                acc[t] = mfma32(a, *(const s16x8 *)(s_x + xoff[t] + rx), acc[t]);
+        }
     }
     // D[row = co tile row 4 grp + i][col = lane % 16]
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = (int)(cot * 16u + 4u * grp + (uint32_t)i);
-        if (r >= cout || !tok) continue;
-        const size_t o = ((size_t)tap * cout + r) * cin + ci;
-        atomicAdd(dw + o, acc[i]);
+    for (int t = 0; t < NT; ++t) {
+        const int q = (int)wave * NT + t;
+        const int tap = CIN4 ? q * 4 + (int)(m >> 2) : q;
+        const int ci = CIN4 ? (int)(m & 3u) : (int)(cit * 16u + m);
+        if (!tok[t] || ci >= cin_real) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int co = (int)(cot * 16u + 4u * grp + (uint32_t)i);
+            atomicAdd(dw + ((size_t)tap * cout + co) * cin_real + ci, acc[t][i]);
+        }
     }
 }
 
 int launch_conv_wgrad(hipStream_t s, const NetGeom &g, const uint16_t *x, int cin, const uint16_t *dz,
-                      int cout, float *dw)
+                      int cout, float *dw, int cin_real)
 {
-    const uint32_t V = g.nx * g.ny * g.nz;
-    const uint32_t nchunk = (V + WG_VOX - 1) / WG_VOX;
-    const uint32_t nco = (uint32_t)(cout + 15) / 16u;
-    if (cin == 4) {
-        const uint32_t jobs = 7u * nco * nchunk;
-        hipLaunchKernelGGL(k_conv_wgrad<true>, dim3((jobs + 3u) / 4u), dim3(256), 0, s, g, x, cin, dz, cout,
-                           dw, 7u, nco, 1u, nchunk);
-    } else {
-        if (cin % 16) return -1;
-        const uint32_t nci = (uint32_t)cin / 16u;
-        const uint32_t jobs = 27u * nco * nci * nchunk;
-        hipLaunchKernelGGL(k_conv_wgrad<false>, dim3((jobs + 3u) / 4u), dim3(256), 0, s, g, x, cin, dz,
-                           cout, dw, 27u, nco, nci, nchunk);
-    }
+    if (cout % 16 || (cin != 4 && cin % 16)) return -1;
+    const uint32_t ntx = (g.nx + WT_X - 1) / WT_X, nty = (g.ny + WT_Y - 1) / WT_Y;
+    const uint32_t ntiles = ntx * nty * ((g.nz + WT_Z - 1) / WT_Z);
+    const uint32_t nci = cin == 4 ? 1u : (uint32_t)cin / 16u, pairs = nci * (uint32_t)cout / 16u;
+    const uint32_t aim = cin == 4 ? WT_BLOCKS_IN : WT_BLOCKS;
+    const uint32_t per = (ntiles * pairs + aim - 1u) / aim;
+    const uint32_t nchunk = (ntiles + per - 1u) / per;
+    if (cin == 4)
+        hipLaunchKernelGGL(k_conv_wgrad<true>, dim3(nchunk * pairs), dim3(256), 0, s, g, x, cin, dz, cout, dw,
+                           cin_real, ntx, nty, ntiles, per, nci, nchunk);
+    else
+        hipLaunchKernelGGL(k_conv_wgrad<false>, dim3(nchunk * pairs), dim3(256), 0, s, g, x, cin, dz, cout, dw,
+                           cin_real, ntx, nty, ntiles, per, nci, nchunk);
     return 0;
-}
-
-// db[c] += sum_v dz[v][c] for c < c_real (dz has c_stride <= 256
-// channels); one block per 1024 voxels, threads over (voxel lane, channel)
-// so that a block reads dz rows contiguously, partial sums folded in LDS
-__global__ void __launch_bounds__(256) k_bias_grad(uint32_t V, const uint16_t *__restrict__ dz, int c_stride,
-                                                   int c_real, float *__restrict__ db)
-{
-    __shared__ float part[256];
-    const uint32_t C = (uint32_t)c_stride;
-    const uint32_t lanes = 256u / C;
-    const uint32_t ch = threadIdx.x % C, vl = threadIdx.x / C;
-    const uint32_t v0 = blockIdx.x * 1024u;
-    const uint32_t ve = v0 + 1024u < V ? v0 + 1024u : V;
-    float sum = 0.f;
-    if (vl < lanes)
-        for (uint32_t v = v0 + vl; v < ve; v += lanes) sum += bf2f(dz[(size_t)v * C + ch]);
-    part[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x < C && (int)threadIdx.x < c_real) {
-        float t = 0.f;
-        for (uint32_t k = 0; k < lanes; ++k) t += part[k * C + threadIdx.x];
-        atomicAdd(db + threadIdx.x, t);
-    }
-}
-
-void launch_bias_grad(hipStream_t s, uint32_t V, const uint16_t *dz, int c_stride, int c_real, float *db)
-{
-    hipLaunchKernelGGL(k_bias_grad, dim3((V + 1023u) / 1024u), dim3(256), 0, s, V, dz, c_stride, c_real, db);
 }
 
 // ---------------------------------------------------------------------------
@@ -890,28 +916,53 @@ void launch_up_bwd(hipStream_t s, const NetGeom &gc, const float *dfine, int c, 
     hipLaunchKernelGGL(k_up_bwd, dim3((n + 255u) / 256u), dim3(256), 0, s, gc, dfine, c, dcoarse);
 }
 
-// dz = dy where the ReLU output y > 0, else 0, as BF16 with cpad channels
-// (channels c .. cpad-1 are zero)
+// dz = dy where the ReLU output y > 0, else 0, as BF16, and db[c] += sum_v
+// dz[v][c] of the rounded values; C channels, a multiple of 4 up to 64.  A
+// block takes `vpb` consecutive voxels, four channels per thread, and folds
+// its sums in LDS.
 __global__ void __launch_bounds__(256) k_relu_mask(uint32_t V, const float *__restrict__ dy,
-                                                   const uint16_t *__restrict__ y, int c, int cpad,
-                                                   uint16_t *__restrict__ dz)
+                                                   const uint16_t *__restrict__ y, uint32_t C, uint32_t vpb,
+                                                   uint16_t *__restrict__ dz, float *__restrict__ db)
 {
-    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
-    if (idx >= V * (uint32_t)cpad) return;
-    const uint32_t v = idx / (uint32_t)cpad, ch = idx % (uint32_t)cpad;
-    float r = 0.f;
-    if ((int)ch < c) {
-        const size_t i = (size_t)v * c + ch;
-        r = (y == nullptr || bf2f(y[i]) > 0.f) ? dy[i] : 0.f;
+    __shared__ float part[256][4];
+    const uint32_t q = C / 4u, lanes = 256u / q;
+    const uint32_t c4 = threadIdx.x % q, vl = threadIdx.x / q;
+    const uint32_t v0 = blockIdx.x * vpb;
+    const uint32_t ve = v0 + vpb < V ? v0 + vpb : V;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    if (vl < lanes)
+        for (uint32_t v = v0 + vl; v < ve; v += lanes) {
+            const size_t i = (size_t)v * C + 4u * c4;
+            const f32x4 d = *(const f32x4 *)(dy + i);
+            const bf16x4 a = *(const bf16x4 *)(y + i);
+            bf16x4 r;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint16_t b = f2bf(bf2f((uint16_t)a[k]) > 0.f ? d[k] : 0.f);
+                r[k] = (short)b;
+                sum[k] += bf2f(b);
+            }
+            *(bf16x4 *)(dz + i) = r;
+        }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[threadIdx.x][k] = sum[k];
+    __syncthreads();
+    if (threadIdx.x < C) {
+        float t = 0.f;
+        for (uint32_t l = 0; l < lanes; ++l) t += part[l * q + threadIdx.x / 4u][threadIdx.x & 3u];
+        atomicAdd(db + threadIdx.x, t);
     }
-    dz[idx] = f2bf(r);
 }
 
-void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t *y, int c, int cpad,
-                      uint16_t *dz)
+void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t *y, int c, uint16_t *dz,
+                      float *db)
 {
-    const uint32_t n = V * (uint32_t)cpad;
-    hipLaunchKernelGGL(k_relu_mask, dim3((n + 255u) / 256u), dim3(256), 0, s, V, dy, y, c, cpad, dz);
+    // at least one voxel per thread, at most 512 blocks (two per compute unit)
+    const uint32_t lanes = 256u / ((uint32_t)c / 4u);
+    uint32_t vpb = (V + 511u) / 512u;
+    if (vpb < lanes) vpb = lanes;
+    hipLaunchKernelGGL(k_relu_mask, dim3((V + vpb - 1u) / vpb), dim3(256), 0, s, V, dy, y, (uint32_t)c, vpb, dz,
+                       db);
 }
 
 // FP32 -> BF16 with channel padding: out[v][cpad] from in[v][c]
@@ -930,75 +981,55 @@ void launch_to_bf16_pad(hipStream_t s, uint32_t V, const float *in, int c, int c
     hipLaunchKernelGGL(k_to_bf16_pad, dim3((n + 255u) / 256u), dim3(256), 0, s, V, in, c, cpad, out);
 }
 
-// Pack one layer's FP32 parameters (w[27][cout][cin] then b[cout]) into
-// the BF16 operand layouts: forward wf[27][cout_pad][cin_pad] and, for the
-// data gradient (the adjoint: taps mirrored, channels swapped),
-// wt[27][cin_pad2][cout_pad2] with wt[tap][ci][co] = w[26 - tap][co][ci].
-__global__ void __launch_bounds__(256) k_pack_weights(const float *__restrict__ w, int cin, int cout,
-                                                      uint16_t *__restrict__ wf, int cin_pad, int cout_pad,
-                                                      uint16_t *__restrict__ wt, int tin_pad, int tout_pad)
+// Pack FP32 parameters (w[27][cout][cin] of each layer) into the BF16
+// operand layouts: forward wf[27][cout_pad][cin_pad] and, for the data
+// gradient (the adjoint: taps mirrored, channels swapped),
+// wt[27][cin_pad2][cout_pad2] with wt[tap][ci][co] = w[26 - tap][co][ci].  One
+// launch for all layers, and for the conversion of the network's input (in,
+// rows of 3, to BF16 rows of 4; null: none), which the packing does not need:
+// nine launches of 3 us took a quarter of a forward pass.
+__global__ void __launch_bounds__(256) k_pack_weights(PackLayers p)
 {
-    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t nf = 27u * (uint32_t)cout_pad * (uint32_t)cin_pad;
-    if (idx < nf) {
-        const uint32_t ci = idx % (uint32_t)cin_pad;
-        const uint32_t r = idx / (uint32_t)cin_pad;
-        const uint32_t co = r % (uint32_t)cout_pad, tap = r / (uint32_t)cout_pad;
-        wf[idx] = ((int)ci < cin && (int)co < cout) ? f2bf(w[((size_t)tap * cout + co) * cin + ci]) : (uint16_t)0;
+    int l = 0;
+    while (l < p.n && blockIdx.x >= p.layer[l].blocks) ++l;
+    const uint32_t b0 = l ? p.layer[l - 1].blocks : 0u;
+    const uint32_t idx = (blockIdx.x - b0) * 256u + threadIdx.x;
+    if (l == p.n) {
+        if (idx >= p.V) return;
+        const float *r = p.in + 3 * (size_t)idx;
+        const bf16x4 o = {(short)f2bf(r[0]), (short)f2bf(r[1]), (short)f2bf(r[2]), 0};
+        *(bf16x4 *)(p.in4 + 4 * (size_t)idx) = o;
+        return;
     }
-    if (wt == nullptr) return;
-    const uint32_t nt = 27u * (uint32_t)tout_pad * (uint32_t)tin_pad;
-    if (idx < nt) {
+    const PackLayer &L = p.layer[l];
+    const uint32_t cin = (uint32_t)L.cin, cout = (uint32_t)L.cout;
+    if (idx < 27u * (uint32_t)L.cout_pad * (uint32_t)L.cin_pad) {
+        const uint32_t ci = idx % (uint32_t)L.cin_pad;
+        const uint32_t r = idx / (uint32_t)L.cin_pad;
+        const uint32_t co = r % (uint32_t)L.cout_pad, tap = r / (uint32_t)L.cout_pad;
+        L.wf[idx] = (ci < cin && co < cout) ? f2bf(L.w[((size_t)tap * cout + co) * cin + ci]) : (uint16_t)0;
+    }
+    if (L.wt && idx < 27u * (uint32_t)L.tout_pad * (uint32_t)L.tin_pad) {
         // wt layout [tap][new co = ci][new ci = co]
-        const uint32_t nci = idx % (uint32_t)tin_pad;      // original output channel
-        const uint32_t r = idx / (uint32_t)tin_pad;
-        const uint32_t nco = r % (uint32_t)tout_pad, tap = r / (uint32_t)tout_pad;  // nco: original input channel
-        wt[idx] = ((int)nci < cout && (int)nco < cin)
-                      ? f2bf(w[((size_t)(26u - tap) * cout + nci) * cin + nco])
-                      : (uint16_t)0;
+        const uint32_t nci = idx % (uint32_t)L.tin_pad;      // original output channel
+        const uint32_t r = idx / (uint32_t)L.tin_pad;
+        const uint32_t nco = r % (uint32_t)L.tout_pad, tap = r / (uint32_t)L.tout_pad;  // original input channel
+        L.wt[idx] = (nci < cout && nco < cin) ? f2bf(L.w[((size_t)(26u - tap) * cout + nci) * cin + nco])
+                                              : (uint16_t)0;
     }
 }
 
-void launch_pack_weights(hipStream_t s, const float *w, int cin, int cout, uint16_t *wf, int cin_pad,
-                         int cout_pad, uint16_t *wt, int tin_pad, int tout_pad)
+void launch_pack_weights(hipStream_t s, PackLayers &p)
 {
-    uint32_t n = 27u * (uint32_t)cout_pad * (uint32_t)cin_pad;
-    const uint32_t n2 = 27u * (uint32_t)tout_pad * (uint32_t)tin_pad;
-    if (wt && n2 > n) n = n2;
-    hipLaunchKernelGGL(k_pack_weights, dim3((n + 255u) / 256u), dim3(256), 0, s, w, cin, cout, wf, cin_pad,
-                       cout_pad, wt, tin_pad, tout_pad);
-}
-
-// Add a padded FP32 weight gradient gw[27][cout_pad][cin_pad] into the
-// flat layout g[27][cout][cin].
-__global__ void __launch_bounds__(256) k_unpack_wgrad(const float *__restrict__ gw, int cin, int cin_pad,
-                                                      int cout, int cout_pad, float *__restrict__ g)
-{
-    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t n = 27u * (uint32_t)cout * (uint32_t)cin;
-    if (idx >= n) return;
-    const uint32_t ci = idx % (uint32_t)cin;
-    const uint32_t r = idx / (uint32_t)cin;
-    const uint32_t co = r % (uint32_t)cout, tap = r / (uint32_t)cout;
-    g[idx] += gw[((size_t)tap * cout_pad + co) * cin_pad + ci];
-}
-
-void launch_unpack_wgrad(hipStream_t s, const float *gw, int cin, int cin_pad, int cout, int cout_pad,
-                         float *g)
-{
-    const uint32_t n = 27u * (uint32_t)cout * (uint32_t)cin;
-    hipLaunchKernelGGL(k_unpack_wgrad, dim3((n + 255u) / 256u), dim3(256), 0, s, gw, cin, cin_pad, cout,
-                       cout_pad, g);
-}
-
-__global__ void __launch_bounds__(256) k_fill_f32(float *__restrict__ p, size_t n, float v)
-{
-    const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-void launch_fill_f32(hipStream_t s, float *p, size_t n, float v)
-{
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_fill_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
+    uint32_t at = 0;
+    for (int l = 0; l < p.n; ++l) {
+        PackLayer &L = p.layer[l];
+        uint32_t n = 27u * (uint32_t)L.cout_pad * (uint32_t)L.cin_pad;
+        const uint32_t n2 = 27u * (uint32_t)L.tout_pad * (uint32_t)L.tin_pad;
+        if (L.wt && n2 > n) n = n2;
+        at += (n + 255u) / 256u;
+        L.blocks = at;
+    }
+    if (p.in) at += (p.V + 255u) / 256u;
+    hipLaunchKernelGGL(k_pack_weights, dim3(at), dim3(256), 0, s, p);
 }
