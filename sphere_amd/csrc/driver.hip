@@ -3080,11 +3080,14 @@ int sph_ensemble_step(sph_ensemble *e, int nsteps)
                 hashed = true;
             }
         }
-        if (hashed || e->phase == 1) {
-            ens_enqueue_phase(e, e->ph[e->phase]);
-            ens_advance_all(e);
-            --left;
-        }
+        // a step of its own after a hash, and another where the plan's second
+        // phase is due: the pairs below begin with its first
+        for (int q = 0; q < 2 && left > 0; ++q)
+            if (q == 0 ? hashed : e->phase == 1) {
+                ens_enqueue_phase(e, e->ph[e->phase]);
+                ens_advance_all(e);
+                --left;
+            }
         if (left >= 2 && e->use_graph && !e->exec) {
             HIPCHK_E(hipStreamSynchronize(e->stream));
             if ((rc = ens_capture(e))) {
