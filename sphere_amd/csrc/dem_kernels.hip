@@ -1567,8 +1567,6 @@ __device__ __forceinline__ void topology_lists_body(
     const float *__restrict__ nl_disp, uint32_t *__restrict__ flags_rw, uint32_t cur,
     uint32_t gpw, uint32_t bid, uint32_t nblk)
 {
-    // the list rebuild before it did not finish (its grid barrier timed out)
-    if ((*err & ERRF_BARRIER) != 0u) return;
     const uint32_t *flags = flags_rw;
     __shared__ double4 s_x[TW];
     __shared__ int s_g[TW][3];
@@ -1582,21 +1580,31 @@ __device__ __forceinline__ void topology_lists_body(
     const int NCS = (int)a.nc;
     const bool valid = lane < gpw && pos < np;
     const uint32_t a_orig = valid ? pos : 0u;  // lists are by original index
+    // everything that most waves read, requested together: few of their grains
+    // have an entry to test, and trips to memory one after another are then
+    // most of a wave's time
+    const uint32_t bad = *err & ERRF_BARRIER;
+    uint32_t cc = cellc[a_orig], lcnt = nl_cnt[a_orig];
+    const uint32_t fl_step = flags[cur], fl_ovf = flags[NLF_STICKY];
+    const float disp = nl_disp[a_orig], gmin = nl_gmin[a_orig];
+    const double dmax = dmax_since_rebuild(flags);
+    asm volatile("" : : "v"(bad), "v"(cc), "v"(lcnt), "v"(fl_step), "v"(fl_ovf), "v"(disp), "v"(gmin));
+    // the list rebuild before it did not finish (its grid barrier timed out)
+    if (bad) return;
     // this step's cell from the hash (all ones outside the grid)
-    const uint32_t cc = valid ? cellc[pos] : 0xffffffffu;
+    if (!valid) cc = 0xffffffffu;
     const bool inside = cc != 0xffffffffu;
     if (valid && !inside) atomicOr(err, ERRF_GRID);
     const int gx = (int)(cc & 2047u), gy = (int)((cc >> 11) & 2047u), gz = (int)(cc >> 22);
-    const uint32_t lcnt = inside ? nl_cnt[pos] : 0u;
+    if (!inside) lcnt = 0u;
     const bool list_ovf = lcnt == NL_OVF;
     // Entries to test.  On steps that rebuilt the lists, or on which a grain
     // wrapped around a periodic boundary (images may change), every entry.
     // Otherwise the row can only change by a new contact: an entry not in the
     // row whose surface gap at the rebuild is at most twice the largest
     // displacement since then (plus a rounding margin).
-    const bool full = (flags[cur] & (NLF_REBUILD | NLF_WRAP)) != 0u || flags[NLF_STICKY] != 0u;
+    const bool full = (fl_step & (NLF_REBUILD | NLF_WRAP)) != 0u || fl_ovf != 0u;
     if (full && bid == 0 && lane == 0) flags_rw[NLF_FULL] += 1u;
-    const double dmax = dmax_since_rebuild(flags);
     Set128 q = {0ull, 0ull};
     uint32_t n = 0;
     if (!list_ovf && lcnt > 0) {
@@ -1611,10 +1619,10 @@ __device__ __forceinline__ void topology_lists_body(
             // up to float, as the stored gaps are rounded down, with a margin
             // for the rounding of the displacements themselves.
             const double marg = 1e-11 * (g.L[0] + g.L[1] + g.L[2]);
-            const double da = (double)nl_disp[pos];
+            const double da = (double)disp;
             const float thr = __double2float_ru((da + sqrt(dmax)) * (1.0 + 1e-9) + marg);
             // nl_gmin bounds the gaps of the entries not in the row
-            if (!(nl_gmin[pos] > thr)) {
+            if (!(gmin > thr)) {
                 // eight entries per iteration, their loads issued together
                 for (uint32_t k0 = 0; k0 < lcnt; k0 += 8) {
                     uint8_t sl[8];
@@ -1903,8 +1911,6 @@ __device__ __forceinline__ void forces_body(
     const float *__restrict__ nl_gap, float *__restrict__ nl_gmin,
     const uint32_t *__restrict__ err, uint32_t gpw, uint32_t bid, uint32_t nblk)
 {
-    // list mode: the list rebuild of this step did not finish
-    if (err && (*err & ERRF_BARRIER) != 0u) return;
     __shared__ uint32_t s_a[FW];
     __shared__ uint8_t s_own[FW], s_slot[FW], s_rm[FW], s_rmk[FW];
     __shared__ double s_rec[NREC][FW];
@@ -1915,7 +1921,12 @@ __device__ __forceinline__ void forces_body(
     const uint32_t np = a.np;
     const bool valid = lane < gpw && pos < np;
     const uint32_t a_orig = valid ? (order ? order[pos] : pos) : 0u;
-    const uint64_t mask = valid ? cmask[a_orig] : 0ull;
+    const uint32_t bad = err ? *err & ERRF_BARRIER : 0u;
+    uint64_t mask = cmask[a_orig];
+    asm volatile("" : : "v"(bad), "v"(mask));  // both requested before either is needed
+    // list mode: the list rebuild of this step did not finish
+    if (bad) return;
+    if (!valid) mask = 0ull;
     const uint32_t n = (uint32_t)__popcll(mask);
     // exclusive scan of the row sizes over the wave
     uint32_t incl = n;
