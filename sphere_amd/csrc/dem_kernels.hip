@@ -632,8 +632,8 @@ void launch_nl_build(hipStream_t s, const StepArgs &a, const NLArgs &n, const De
 // flag and return, and each such launch still costs its dispatch.  On the
 // list path the radix passes, the cell clear and the reorder run as one
 // kernel whose phases are separated by grid barriers, and the list build
-// follows as one more launch; a step without a rebuild then costs two
-// dispatches instead of nine.  The grid is at most one block per compute
+// follows as one more launch (in small boxes it joins the kernel); a step
+// without a rebuild then costs two dispatches, or one, instead of nine.  The grid is at most one block per compute
 // unit, so every block is resident.
 
 // Grid barrier.  bar[0] counts arrivals, bar[1] is the generation; `gen` is

@@ -5,8 +5,8 @@
 // (src/main.cpp:28-225).  One context owns one device arena and one HIP
 // stream; all kernels of a step are enqueued back to back on that stream
 // (the reference synchronises after every launch).  The host waits only
-// where the algorithm needs a device value: the Darcy convergence check every
-// 10 sweeps, output events, and the end of each call.
+// where the algorithm needs a device value: the outcome of a fluid solve,
+// output events, and the end of each call.
 #include <hip/hip_runtime.h>
 
 #include "net.h"
@@ -583,7 +583,7 @@ static int upload(sph_ctx *ctx)
             ctx->rb_blocks = 0;
             ctx->rb_cap = 0;
             int cus = 0;
-            // (a fluid run rebuilds every step: there the separate launches,
+            // (a fluid run sorts every step: there the separate launches,
             // on full grids, are faster; its barrier words serve the
             // multi-box launches of an ensemble)
             if (ctx->rb_fused && rebuild_blocks_per_cu() > 0 &&

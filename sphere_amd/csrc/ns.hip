@@ -20,6 +20,8 @@
 //     (src/navierstokes.cpp:275-297).  Once a test passes, the iterations
 //     already enqueued return at once; the host reads the outcome after
 //     each batch of about 100 iterations.
+// Where the grid and the boundaries allow it, all iterations of a solve run in
+// one resident launch instead (NsOp, resident.h), with the same values.
 // Where the reference's ghost kernel races (bc_bot = 2 or bc_top = 2), the
 // ghost layer below z = 0 keeps the bottom rule's value and the layer above
 // z = nz-1 the top rule's; smoothing reads the field as it was before the
