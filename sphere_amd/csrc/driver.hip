@@ -633,11 +633,14 @@ struct ReadRow {
 // moved a 1,000,000-grain state at 7 GB/s (30 ms), because one thread copies
 // out of the driver's staging buffer and takes the page faults of a
 // destination that has not been touched.  Here READ_THREADS threads move
-// pieces of READ_PIECE bytes, each through a staging piece of its own.  A state
+// pieces, each through a staging piece of its own.  A state
 // that fits into the staging memory at once, up to READ_SMALL, is copied with
 // one wait and no threads (0.6 ms for 1,000 grains with a wait per array).
 #define READ_THREADS 8
-#define READ_PIECE (size_t(2) << 20)
+// A piece is 1/32 of the state, 512 KB to 2 MB: 2 MB ones take each of many
+// small boxes 1 ms to make, 512 KB ones cost a 224 MB state 4 ms per read.
+#define READ_PIECE_MIN (size_t(512) << 10)
+#define READ_PIECE_MAX (size_t(2) << 20)
 #define READ_SMALL (size_t(4) << 20)
 static int read_rows(sph_ctx *ctx, const std::vector<ReadRow> &rows)
 {
@@ -645,7 +648,8 @@ static int read_rows(sph_ctx *ctx, const std::vector<ReadRow> &rows)
     for (const ReadRow &r : rows) total += (r.bytes + 255) / 256 * 256;
     if (!total) return SPH_OK;
     const bool small = total <= READ_SMALL;
-    const size_t cap = small ? total : READ_THREADS * READ_PIECE;
+    const size_t piece = std::min(READ_PIECE_MAX, std::max(READ_PIECE_MIN, total / 32 / 4096 * 4096));
+    const size_t cap = small ? total : READ_THREADS * piece;
     if (ctx->read_cap < cap) {
         if (ctx->read_pin) (void)hipHostFree(ctx->read_pin);
         ctx->read_pin = nullptr;
@@ -669,15 +673,15 @@ static int read_rows(sph_ctx *ctx, const std::vector<ReadRow> &rows)
     }
     std::vector<ReadRow> pieces;
     for (const ReadRow &r : rows)
-        for (size_t o = 0; o < r.bytes; o += READ_PIECE)
-            pieces.push_back(ReadRow{(char *)r.dst + o, (const char *)r.src + o, std::min(READ_PIECE, r.bytes - o)});
+        for (size_t o = 0; o < r.bytes; o += piece)
+            pieces.push_back(ReadRow{(char *)r.dst + o, (const char *)r.src + o, std::min(piece, r.bytes - o)});
     hipEvent_t ev[READ_THREADS] = {};
     hipError_t err[READ_THREADS];
     for (int t = 0; t < READ_THREADS; ++t) err[t] = hipEventCreateWithFlags(&ev[t], hipEventDisableTiming);
     auto work = [&](int t) {
         hipError_t e = err[t];
         if (e == hipSuccess) e = hipSetDevice(ctx->device);
-        char *pin = ctx->read_pin + (size_t)t * READ_PIECE;
+        char *pin = ctx->read_pin + (size_t)t * piece;
         for (size_t k = (size_t)t; k < pieces.size() && e == hipSuccess; k += READ_THREADS) {
             e = hipMemcpyAsync(pin, pieces[k].src, pieces[k].bytes, hipMemcpyDeviceToHost, ctx->stream);
             if (e == hipSuccess) e = hipEventRecord(ev[t], ctx->stream);
