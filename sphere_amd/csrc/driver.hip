@@ -1483,7 +1483,10 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
             if (rc) return rc;
         }
     } else if (ctx->db.clock) {
-        launch_step_end(s, step_args(ctx), ctx->db);
+        // without grains the walls stay where they are: only the clock advances
+        StepArgs a = step_args(ctx);
+        a.walls.nw = 0;
+        launch_step_end(s, a, ctx->db);
     }
     h.time_current += h.time_dt;
     ctx->filetimeclock += h.time_dt;
