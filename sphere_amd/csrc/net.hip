@@ -82,6 +82,8 @@ struct sph_net {
     // gradients (FP32) and the BF16 operand of the weight gradient
     float *d_h0, *d_y0, *d_a1, *d_y1, *d_a2, *d_y2, *d_a3, *d_x3, *d_p2, *d_p1, *d_p0;
     uint16_t *dz;
+    // the gradient of one backward pass; zero between passes
+    float *grad;
 };
 
 static bool net_alloc(sph_net *n, void **p, size_t bytes)
@@ -173,6 +175,8 @@ sph_net *sph_net_create(int device, uint32_t nx, uint32_t ny, uint32_t nz, uint3
     A32(&n->d_p2, (size_t)V[3] * 48); A32(&n->d_p1, (size_t)V[2] * 32);
     A32(&n->d_p0, (size_t)V[1] * 16);
     A16(&n->dz, (size_t)V[0] * 16);
+    A32(&n->grad, off);
+    ok = ok && hipMemset(n->grad, 0, off * 4) == hipSuccess && hipDeviceSynchronize() == hipSuccess;
     (void)hipSetDevice(prev);
     if (!ok) {
         g_net_error = "device allocation failed";
@@ -403,7 +407,11 @@ int sph_net_forward(sph_net *n, const float *params, const float *input, float *
 }
 
 // Backward pass of the last forward: grad_output[V0] FP32 (dLoss/dout);
-// adds dLoss/dparams into grad_params (FP32, param_count values).
+// adds dLoss/dparams into grad_params (FP32, param_count values).  The layers
+// sum into a buffer that starts at zero, which is added once: a caller who
+// accumulates passes gets one rounding at the size of the accumulated value,
+// not one per block (up to 512).  The launch makes a forward and backward pass
+// on 48 x 48 x 96 cells 9 us longer (412 to 421 us).
 int sph_net_backward(sph_net *n, const float *params, const float *grad_output, float *grad_params,
                      void *stream)
 {
@@ -421,11 +429,11 @@ int sph_net_backward(sph_net *n, const float *params, const float *grad_output, 
     // channels)
     auto wgrad = [&](int l, const float *dy, const uint16_t *y, const uint16_t *x, int cin_x, int level) {
         const LayerSpec &L = kLayers[l];
-        launch_relu_mask(s, V[level], dy, y, L.cout, n->dz, grad_params + n->boff[l]);
-        rc |= launch_conv_wgrad(s, g[level], x, cin_x, n->dz, L.cout, grad_params + n->woff[l], L.cin);
+        launch_relu_mask(s, V[level], dy, y, L.cout, n->dz, n->grad + n->boff[l]);
+        rc |= launch_conv_wgrad(s, g[level], x, cin_x, n->dz, L.cout, n->grad + n->woff[l], L.cin);
     };
     // c8: out = w8 . h0 + b8 (weights and bias contiguous)
-    launch_proj_bwd(s, V[0], grad_output, n->h0, params + n->woff[8], n->d_h0, grad_params + n->woff[8]);
+    launch_proj_bwd(s, V[0], grad_output, n->h0, params + n->woff[8], n->d_h0, n->grad + n->woff[8]);
     // c7: h0 = relu(conv(y0))
     wgrad(7, n->d_h0, n->h0, n->y0, 16, 0);
     rc |= launch_conv_fwd(s, g[0], n->dz, 16, n->wt[7], 16, nullptr, 16, n->d_y0, NET_OUT_F32);
@@ -456,6 +464,7 @@ int sph_net_backward(sph_net *n, const float *params, const float *grad_output, 
     launch_pool_bwd(s, g[0], n->d_p0, 16, n->d_y0);
     // c0: x0 = relu(conv(in))
     wgrad(0, n->d_y0, n->x0, n->in4, 4, 0);
+    launch_add_and_clear(s, sph_net_param_count(), n->grad, grad_params);
     if (rc) {
         g_net_error = "unsupported layer shape";
         return SPH_ERR_VALUE;

@@ -53,6 +53,8 @@ void launch_up_bwd(hipStream_t s, const NetGeom &gc, const float *dfine, int c, 
 // dz = bf16(dy where y > 0), db += sum_v dz; c a multiple of 4 up to 64
 void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t *y, int c, uint16_t *dz,
                       float *db);
+// dst += src, src = 0
+void launch_add_and_clear(hipStream_t s, size_t n, float *src, float *dst);
 void launch_to_bf16_pad(hipStream_t s, uint32_t V, const float *in, int c, int cpad, uint16_t *out);
 struct PackLayer {
     const float *w;

@@ -965,6 +965,20 @@ void launch_relu_mask(hipStream_t s, uint32_t V, const float *dy, const uint16_t
                        db);
 }
 
+// (an atomic add: passes of several networks may add to one dst)
+__global__ void __launch_bounds__(256) k_add_and_clear(size_t n, float *__restrict__ src, float *__restrict__ dst)
+{
+    const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    atomicAdd(dst + i, src[i]);
+    src[i] = 0.f;
+}
+
+void launch_add_and_clear(hipStream_t s, size_t n, float *src, float *dst)
+{
+    hipLaunchKernelGGL(k_add_and_clear, dim3((unsigned)((n + 255u) / 256u)), dim3(256), 0, s, n, src, dst);
+}
+
 // FP32 -> BF16 with channel padding: out[v][cpad] from in[v][c]
 __global__ void __launch_bounds__(256) k_to_bf16_pad(uint32_t V, const float *__restrict__ in, int c,
                                                      int cpad, uint16_t *__restrict__ out)
