@@ -209,10 +209,27 @@ int sph_set_rebuild_kernel(sph_ctx *ctx, int fused);
  * that runs past it ends the kernel on every block, the list and contact
  * kernels after it skip their work, and the step returns SPH_ERR_HIP; a
  * small bound forces that path from the host, for tests of the failure
- * handling.  It also bounds the polls of a fluid's resident iterations
- * (default 2^20); where one runs out the solve is repeated with one launch
- * per sweep, as are the later ones.  Takes effect at once. */
+ * handling.  It also sets the bound of sph_set_resident_wait_limit from sweep
+ * 0 on.  Takes effect at once. */
 int sph_set_barrier_spin_limit(sph_ctx *ctx, uint32_t sleeps);
+
+/* The fluids' resident launches: one launch runs many Jacobi sweeps of a
+ * solve, its blocks waiting for each other's halo values.  No counterpart in
+ * the reference.  The limit bounds those waits, in polls, for the launches that
+ * begin at sweep from_sweep of a solve or later (0: the default, 2^20, about a
+ * second).  Where a wait runs out, the solve is repeated with one launch per
+ * sweep, to the same bits, as are the later ones.  A small bound forces that
+ * path from the host.  It holds for the context's Darcy fluid and for an
+ * attached Navier-Stokes fluid; takes effect at once. */
+int sph_set_resident_wait_limit(sph_ctx *ctx, uint32_t polls, uint32_t from_sweep);
+
+/* How the solves of the loaded state's Darcy fluid ran (sph_ns_get_resident_stats:
+ * those of a Navier-Stokes fluid since its creation). */
+typedef struct sph_resident_stats {
+    uint64_t solves;              /* solved in resident launches */
+    uint64_t repeated;            /* repeated because a wait ran out */
+} sph_resident_stats;
+int sph_get_resident_stats(sph_ctx *ctx, sph_resident_stats *out);
 
 /* Load a state: replaces DEM::readbin + checkValues + transfer to the device
  * (src/file_io.cpp:30-417, src/sphere.cpp:145-345, src/device.cu:667-752).
@@ -468,6 +485,7 @@ int sph_ns_read(sph_ns *ns, double *v, double *p, double *phi, double *dphi);
  * v_z ((nx+3)(ny+3)(nz+3) each), 3 epsilon ((nx+2)(ny+2)(nz+2)). */
 int sph_ns_read_field(sph_ns *ns, int which, double *dst);
 int sph_ns_get_stats(const sph_ns *ns, sph_ns_stats *out);
+int sph_ns_get_resident_stats(const sph_ns *ns, sph_resident_stats *out);
 /* Grains held in place in the fluid (np = 0 clears them): rows of 4,
  * x = (x, y, z, radius) and vel = (vx, vy, vz, unused), the grid's origin
  * and periodic mode (0 none, 1 x and y, 2 x; src/contactsearch.cuh:12-84).

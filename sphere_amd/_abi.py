@@ -90,6 +90,10 @@ class SphDarcyStats(ctypes.Structure):
                 ("solve_ms", _d), ("corrections", ctypes.c_uint64)]
 
 
+class SphResidentStats(ctypes.Structure):
+    _fields_ = [("solves", ctypes.c_uint64), ("repeated", ctypes.c_uint64)]
+
+
 # Names of the array members and their (dtype, per-item width, count key).
 PARTICLE_ARRAYS = [("x", numpy.float64, 4), ("xyzsum", numpy.float64, 3),
                    ("vel", numpy.float64, 4), ("force", numpy.float64, 3),
@@ -201,6 +205,8 @@ def load_library(path=None):
         "sph_set_neighbor_lists": (ctypes.c_int, [vp, ctypes.c_double, ctypes.c_int]),
         "sph_set_rebuild_kernel": (ctypes.c_int, [vp, ctypes.c_int]),
         "sph_set_barrier_spin_limit": (ctypes.c_int, [vp, ctypes.c_uint32]),
+        "sph_set_resident_wait_limit": (ctypes.c_int, [vp, ctypes.c_uint32, ctypes.c_uint32]),
+        "sph_get_resident_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphResidentStats)]),
         "sph_get_neighbor_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphNeighborStats)]),
         "sph_load_state": (ctypes.c_int, [vp, ctypes.POINTER(SphState)]),
         "sph_load_file": (ctypes.c_int, [vp, ctypes.c_char_p, ctypes.c_int]),
@@ -251,6 +257,7 @@ def load_library(path=None):
         "sph_ns_read": (ctypes.c_int, [vp, _pd, _pd, _pd, _pd]),
         "sph_ns_read_field": (ctypes.c_int, [vp, ctypes.c_int, _pd]),
         "sph_ns_get_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphNsStats)]),
+        "sph_ns_get_resident_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphResidentStats)]),
         "sph_ns_set_grains": (ctypes.c_int, [vp, ctypes.c_uint32, _pd, _pd, _pd, ctypes.c_int32]),
         "sph_ns_read_grain_forces": (ctypes.c_int, [vp, _pd, _pd, _pd, _pd]),
         "sph_ns_attach": (ctypes.c_int, [vp, vp]),
@@ -397,6 +404,17 @@ class Engine:
         """Bound of the list rebuild kernel's grid-barrier waits and of the
         fluid's resident iterations (0: defaults)."""
         self._check(self.lib.sph_set_barrier_spin_limit(self.ctx, int(sleeps)))
+
+    def set_resident_wait_limit(self, polls, from_sweep=0):
+        """Bound in polls of the waits in a fluid's resident launches that
+        begin at sweep from_sweep of a solve or later (0: the default)."""
+        self._check(self.lib.sph_set_resident_wait_limit(self.ctx, int(polls), int(from_sweep)))
+
+    def resident_stats(self):
+        """How the Darcy solves of the loaded state ran."""
+        s = SphResidentStats()
+        self._check(self.lib.sph_get_resident_stats(self.ctx, ctypes.byref(s)))
+        return s
 
     def set_profiling(self, on):
         self._check(self.lib.sph_set_profiling(self.ctx, int(on)))
@@ -608,6 +626,12 @@ class NavierStokes:
     def stats(self):
         st = SphNsStats()
         self._check(self.lib.sph_ns_get_stats(self.h, ctypes.byref(st)))
+        return st
+
+    def resident_stats(self):
+        """How the solves ran."""
+        st = SphResidentStats()
+        self._check(self.lib.sph_ns_get_resident_stats(self.h, ctypes.byref(st)))
         return st
 
     def set_grains(self, x, vel, origo=(0.0, 0.0, 0.0), periodic=1):

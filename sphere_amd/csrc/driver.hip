@@ -86,7 +86,8 @@ struct sph_ctx {
     unsigned long long *h_u64 = nullptr;
     unsigned long long *h_state = nullptr;  // Jacobi solve state (4 words)
     unsigned int jacobi_hint = 0;           // sweeps of the last solve
-    Resident res;                           // tiles and inboxes of the resident sweeps
+    Resident res;                           // tiles and outboxes of the resident sweeps
+    ResidentWait res_wait;                  // the bound of their waits
     double *h_d = nullptr;
     // learned Darcy correction: host parameters, and the network with its
     // device buffers for the loaded grid (made at the first solve)
@@ -922,7 +923,7 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
         const unsigned int len = learned ? (it == 0 ? 2u : 10u) : chunk;
         const unsigned int end = it + std::min(len, h.maxiter - it);
         ResidentArgs a;
-        bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->rb_spin, a);
+        bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->res_wait, a);
         if (ok) {
             ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
             launch_darcy_resident(s, ctx->device, ctx->res, a, da, d, buf[cur], buf[cur ^ 1], h.tolerance);
@@ -942,6 +943,7 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
         const int rc = sync(ctx);
         if (rc) return rc;
         if (!ok || ctx->h_state[0] == RES_ABORT) {
+            if (ctx->h_state[0] == RES_ABORT) ctx->res.repeated++;
             ctx->res.usable = false;
             resident = false;
             launch_darcy_copy_interior(s, da, d.p_old, buf[0]);
@@ -955,6 +957,7 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
     if (ctx->h_state[0] != 0)
         for (k = 0; ends[k] <= ctx->h_state[1];) ++k;
     out = ends.empty() ? 0 : (int)((k + 1) & 1u);
+    ctx->res.solves++;
     return SPH_OK;
 }
 
@@ -1444,7 +1447,7 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
                              (const double *)ctx->db.x_s, ctx->db.cell_start, ctx->db.cell_end, ctx->db.vals,
                              h.origo, h.periodic, (double *)ctx->db.force,
                              h.nw > 0 && (h.wmode[0] == 1 || h.wmode[0] == 3) ? ctx->host_wx0 : -1.0,
-                             ctx->rb_spin, s);
+                             ctx->res_wait, s);
         if (rc) return fail(ctx, rc, sph_ns_last_error());
     }
     if (h.np > 0) {
@@ -1643,6 +1646,21 @@ int sph_set_barrier_spin_limit(sph_ctx *ctx, uint32_t sleeps)
 {
     if (!ctx) return fail(ctx, SPH_ERR_ARG, "null context");
     ctx->rb_spin = sleeps;
+    ctx->res_wait = ResidentWait{sleeps, 0u};
+    return SPH_OK;
+}
+
+int sph_set_resident_wait_limit(sph_ctx *ctx, uint32_t polls, uint32_t from_sweep)
+{
+    if (!ctx) return fail(ctx, SPH_ERR_ARG, "null context");
+    ctx->res_wait = ResidentWait{polls, from_sweep};
+    return SPH_OK;
+}
+
+int sph_get_resident_stats(sph_ctx *ctx, sph_resident_stats *out)
+{
+    if (!ctx || !out) return fail(ctx, SPH_ERR_ARG, "null argument");
+    *out = sph_resident_stats{ctx->res.solves, ctx->res.repeated};
     return SPH_OK;
 }
 

@@ -5,19 +5,19 @@
 #include <cstdint>
 
 #include "../../include/sphere_hip.h"
+#include "resident.h"
 
 // One DEM iteration of the fluid with the context's grains (original-order
 // x and vel rows of 4, the cell sort's sorted x, cell starts and ends and
 // original indices), enqueued on stream s: porosities, the interaction
 // forces (each grain's sum added to force, rows of 3) and, every ndem
 // iterations, the solve (src/device.cu:1213-1898); wall_x >= 0 is the host
-// copy of a top wall's position (wmode 1 or 3), < 0 none; spin bounds the
-// waits of the resident iterations in polls (0: the default).  0 or an
-// SPH_ERR_* code.
+// copy of a top wall's position (wmode 1 or 3), < 0 none; wait bounds the
+// waits of this step's resident iterations.  0 or an SPH_ERR_* code.
 int ns_coupled_step(sph_ns *ns, uint32_t np, const double *x, const double *vel, const double *xs,
                     const uint32_t *cstart, const uint32_t *cend, const uint32_t *gidx,
-                    const double *origo, int periodic, double *force, double wall_x, uint32_t spin,
-                    hipStream_t s);
+                    const double *origo, int periodic, double *force, double wall_x,
+                    const ResidentWait &wait, hipStream_t s);
 // The fluid's grid, to check that it is the context's grid.
 void ns_grid(const sph_ns *ns, uint32_t num[3], double L[3]);
 // Marks the fluid attached to a context (1) or free (0).

@@ -826,8 +826,8 @@ struct sph_ns {
     int cur = 0;
     long iter = 0;
     double t = 0.0;
-    Resident res;           // tiles and inboxes of the resident iterations
-    uint32_t res_spin = 0;  // their wait bound in polls (0: the default)
+    Resident res;           // tiles and outboxes of the resident iterations
+    ResidentWait res_wait;  // the bound of their waits in a coupled step
     double *eps_start = nullptr;  // a solve's start, where it takes several of their launches
     sph_ns_stats st{};
 };
@@ -915,7 +915,7 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
     for (unsigned it = 0; it < P.maxiter; it += std::min(chunk, P.maxiter - it)) {
         ResidentArgs a;
         bool ok = resident_args(n->res, n->s, g.nx, g.ny, g.nz, it, it + std::min(chunk, P.maxiter - it),
-                                n->res_spin, a);
+                                n->res_wait, a);
         if (ok) {
             const NsOp op{g, n->q, n->eps[n->cur], n->eps[1 - n->cur], cv(n->vp), cv(n->vpf), n->phi, n->dphi,
                           n->dst, P.tolerance, n->dp_dz, n->wall0_iz, fixed_div(2.0 * g.dx),
@@ -928,6 +928,7 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
             ok = n->hst->done != RES_ABORT;
         }
         if (!ok) {
+            if (n->hst->done == RES_ABORT) n->res.repeated++;
             n->res.usable = false;
             resident = false;
             n->cur = cur0;
@@ -948,6 +949,7 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
         }
     }
     nijac = converged ? n->hst->conv_nijac + 1 : P.maxiter;
+    n->res.solves++;
     return SPH_OK;
 }
 
@@ -1118,11 +1120,11 @@ int ensure_force_rows(sph_ns *n, uint32_t np)
 
 int ns_coupled_step(sph_ns *n, uint32_t np, const double *x, const double *vel, const double *xs,
                     const uint32_t *cstart, const uint32_t *cend, const uint32_t *gidx,
-                    const double *origo, int periodic, double *force, double wall_x, uint32_t spin,
-                    hipStream_t s)
+                    const double *origo, int periodic, double *force, double wall_x,
+                    const ResidentWait &wait, hipStream_t s)
 {
     n->wall_x = wall_x;
-    n->res_spin = spin;
+    n->res_wait = wait;
     // the fluid's launches go on the context's stream, after its forces
     hipStream_t own = n->s;
     n->s = s;
@@ -1150,6 +1152,7 @@ int ns_coupled_step(sph_ns *n, uint32_t np, const double *x, const double *vel, 
         rc = ns_step_body(n);
     }
     n->s = own;
+    n->res_wait = ResidentWait{};
     return rc;
 }
 
@@ -1442,6 +1445,13 @@ int sph_ns_get_stats(const sph_ns *n, sph_ns_stats *out)
 {
     if (!n || !out) return fail(SPH_ERR_ARG, "bad argument");
     *out = n->st;
+    return SPH_OK;
+}
+
+int sph_ns_get_resident_stats(const sph_ns *n, sph_resident_stats *out)
+{
+    if (!n || !out) return fail(SPH_ERR_ARG, "bad argument");
+    *out = sph_resident_stats{n->res.solves, n->res.repeated};
     return SPH_OK;
 }
 

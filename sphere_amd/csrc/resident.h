@@ -29,7 +29,8 @@
 // state RES_ABORT, every block then leaves, and the host repeats the solve
 // with one launch per sweep.  Blocks of one launch need to be resident
 // together: the grid is at most one block per compute unit, and
-// resident_enqueue() lets the resident launches of a device follow each other.
+// resident_begin() and resident_end() let the resident launches of a device
+// follow each other.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -73,6 +74,13 @@ struct Resident {
     uint32_t tag = 1;                     // next unused tag
     bool usable = false;                  // false: one launch per sweep
     bool planned = false;
+    uint64_t solves = 0;                  // solves whose result came from resident launches
+    uint64_t repeated = 0;                // solves in which a wait ran out
+};
+// The bound of the waits of the launches that begin at iteration `from` or
+// later, in polls (0: RES_SPIN, as for the others).
+struct ResidentWait {
+    uint32_t polls = 0, from = 0;
 };
 // Chooses the tiles of an nx x ny x nz grid on this device; usable stays false
 // where the grid does not fit (see resident.hip).
@@ -81,7 +89,7 @@ void resident_free(Resident &r);
 // The arguments of one launch over iterations [it0, it1); false if the outboxes
 // could not be made.
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,
-                   uint32_t spin, ResidentArgs &out);
+                   const ResidentWait &wait, ResidentArgs &out);
 // Resident launches of one device wait for each other: call before and after
 // the launch.
 void resident_begin(int device, hipStream_t s);

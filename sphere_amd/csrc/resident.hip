@@ -76,7 +76,7 @@ void resident_free(Resident &r)
 }
 
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,
-                   uint32_t spin, ResidentArgs &out)
+                   const ResidentWait &wait, ResidentArgs &out)
 {
     const uint32_t its = it1 - it0;
     if (!r.words_d) {
@@ -101,7 +101,7 @@ bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t 
     out.it1 = it1;
     out.tag0 = r.tag;
     out.box = r.box;
-    out.spin = spin ? spin : RES_SPIN;
+    out.spin = wait.polls && it0 >= wait.from ? wait.polls : RES_SPIN;
     out.mail = r.words_d;
     out.slots = r.words_d + 4u * (size_t)r.tiles * r.box;
     r.tag += its;

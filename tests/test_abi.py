@@ -66,6 +66,7 @@ def struct_fields(name):
                                            ("sph_run_opts", _abi.SphRunOpts),
                                            ("sph_darcy_stats", _abi.SphDarcyStats),
                                            ("sph_neighbor_stats", _abi.SphNeighborStats),
+                                           ("sph_resident_stats", _abi.SphResidentStats),
                                            ("sph_ns_params", _abi.SphNsParams),
                                            ("sph_ns_stats", _abi.SphNsStats)])
 def test_struct_field_order(cname, pyclass):

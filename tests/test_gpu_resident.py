@@ -2,7 +2,9 @@
 oracle: grids at the edges of the tile rules (the smallest, axes shorter than
 a tile, uneven tiles, one and two cells per thread, one grid past the largest
 that fits), periodic and closed z, solves that end at a test and at maxiter;
-and the path a wait that runs out takes, forced by a bound of one poll."""
+and the path a wait that runs out takes, forced by a bound of one poll, in the
+first launch of a solve and in later ones.  Both paths give the same bits, so
+every test reads from the solve statistics which one ran."""
 import numpy
 import pytest
 
@@ -13,6 +15,9 @@ from _ns_oracle import NsOracle
 from _parity import run_pair
 
 pytestmark = pytest.mark.gpu
+
+# cells that fit: 256 compute units, two cells on each of 960 threads
+CELLS = 256 * 2 * 960
 
 
 @pytest.mark.parametrize("shape,bb,bt,maxiter", [
@@ -37,6 +42,8 @@ def test_ns_tiles(shape, bb, bt, maxiter):
         assert numpy.array_equal(gpu.field(3), ora.field(NsOracle.EPS)), step
     for a, b in zip(gpu.read(), ora.read()):
         assert numpy.array_equal(a, b)
+    rs = gpu.resident_stats()
+    assert (rs.solves, rs.repeated) == (2 if numpy.prod(shape) <= CELLS else 0, 0)
     gpu.close()
 
 
@@ -51,6 +58,8 @@ def test_darcy_tiles(nxyz, n, periodic, bc_bot, bc_top, tolerance):
     print("darcy tiles", nxyz, flush=True)
     ora, _ = run_pair(e, s, 2, 2, fluid=True, label="darcy tiles")
     assert e.darcy_stats().sweeps == ora.darcy_stats().sweeps
+    rs = e.resident_stats()
+    assert (rs.solves, rs.repeated) == (4, 0)
     e.close()
 
 
@@ -66,33 +75,74 @@ def test_wait_bound_falls_back():
         print("darcy, wait bound", spin, flush=True)
         e.step(3)
         got.append((e.read().arrays, e.darcy_stats().sweeps))
+        rs = e.resident_stats()
+        assert (rs.solves, rs.repeated) == ((3, 0) if spin == 0 else (0, 1))
         e.close()
     assert got[0][1] == got[1][1]
     for k in ("p_f", "x", "vel", "force"):
         assert numpy.array_equal(got[0][0][k], got[1][0][k]), k
 
 
-def test_ns_wait_bound_falls_back():
+@pytest.mark.parametrize("learned,later", [(True, 2), (True, 12), (True, 22), (False, 20000)])
+def test_wait_bound_in_a_later_launch(learned, later):
+    """A wait that runs out after earlier launches of the solve have written
+    both iterate buffers, with the learned correction between them or past the
+    sweeps of one launch: the repeated solve starts where the first did."""
+    from sphere_amd import learn
+    s = darcy_case(n=700, seed=4, nxyz=(8, 8, 16), tolerance=1e-7 if learned else -1.0,
+                   maxiter=20000 if learned else 20025)
+    s.p_f[:] = 10.0 * numpy.random.default_rng(3).standard_normal(s.p_f.shape)
+    got = []
+    for polls, first in ((0, 0), (1, 0), (1, later)):
+        e = sphere_amd.Engine(0)
+        e.load(s.to_state())
+        e.set_resident_wait_limit(polls, first)
+        if learned:
+            e.set_darcy_net(learn.init_params(1), max_corrections=5)
+        print("darcy, wait bound", polls, "from sweep", first, "learned", learned, flush=True)
+        e.step(1)
+        st, rs = e.darcy_stats(), e.resident_stats()
+        assert (rs.solves, rs.repeated) == ((1, 0) if polls == 0 else (0, 1))
+        assert st.corrections == (5 if learned else 0) and st.sweeps > later
+        got.append((e.read().arrays, st.sweeps, st.corrections, st.last_max_residual))
+        e.close()
+    for g in got[1:]:
+        assert g[1:] == got[0][1:]
+        for k in ("p_f", "x", "vel", "force"):
+            assert numpy.array_equal(got[0][0][k], g[0][k]), k
+
+
+@pytest.mark.parametrize("later", [0, 20000])
+def test_ns_wait_bound_falls_back(later):
+    """In the first launch, and in the one past the 20,000 iterations of a
+    launch, on a column too tall to have converged by then."""
     from _cases import dense_case
     s = dense_case(n=343, seed=4, periodic=1, vmag=0.0, wmag=0.0, spacing_factor=1.1)
+    if later:
+        s.L[2] *= 400.0 / s.num[2]
+        s.num[2] = 400
     nx, ny, nz = (int(v) for v in s.num)
     P = _abi.ns_params(nx, ny, nz, s.L, float(s.time_dt[0]), mu=1.0e-3, rho_f=1000.0, g=s.g,
-                       bc_bot=1, bc_top=0, tolerance=1e-10, maxiter=30000)
+                       bc_bot=1, bc_top=0, tolerance=-1.0 if later else 1e-10, maxiter=20044)
     v = 0.002 * numpy.random.default_rng(6).standard_normal((nx, ny, nz, 3))
     got = []
-    for spin in (0, 1):
-        # the list rebuild's grid barriers have the same bound
-        e = sphere_amd.Engine(0, fused_rebuild=False)
-        e.set_barrier_spin_limit(spin)
+    for polls, first in ((0, 0), (1, later)):
+        e = sphere_amd.Engine(0)
+        e.set_resident_wait_limit(polls, first)
         e.load(s.to_state())
         ns = sphere_amd.NavierStokes(P, v, numpy.zeros((nx, ny, nz)))
         e.attach_fluid(ns)
-        print("ns, wait bound", spin, flush=True)
+        print("ns, wait bound", polls, "from iteration", first, flush=True)
         e.step(3)
-        got.append((ns.read(), ns.stats().iterations, e.read().arrays["vel"]))
+        rs = ns.resident_stats()
+        assert (rs.solves, rs.repeated) == ((3, 0) if polls == 0 else (0, 1))
+        st = ns.stats()
+        assert st.iterations == 3 * 20044 and st.last_max_norm > 0.0 if later else st.iterations < 3 * 20044
+        got.append((ns.read(), (st.iterations, st.last_max_norm), e.read().arrays["vel"]))
         e.attach_fluid(None)
         e.close()
-    assert got[0][1] == got[1][1]
-    for a, b in zip(got[0][0], got[1][0]):
-        assert numpy.array_equal(a, b)
-    assert numpy.array_equal(got[0][2], got[1][2])
+    for g in got[1:]:
+        assert g[1] == got[0][1]
+        for a, b in zip(got[0][0], g[0]):
+            assert numpy.array_equal(a, b)
+        assert numpy.array_equal(got[0][2], g[2])
