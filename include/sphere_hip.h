@@ -228,6 +228,7 @@ int sph_set_resident_wait_limit(sph_ctx *ctx, uint32_t polls, uint32_t from_swee
 typedef struct sph_resident_stats {
     uint64_t solves;              /* solved in resident launches */
     uint64_t repeated;            /* repeated because a wait ran out */
+    uint64_t yielded;             /* one launch per sweep, as list rebuilds of another context ran */
 } sph_resident_stats;
 int sph_get_resident_stats(sph_ctx *ctx, sph_resident_stats *out);
 

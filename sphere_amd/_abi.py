@@ -91,7 +91,7 @@ class SphDarcyStats(ctypes.Structure):
 
 
 class SphResidentStats(ctypes.Structure):
-    _fields_ = [("solves", ctypes.c_uint64), ("repeated", ctypes.c_uint64)]
+    _fields_ = [("solves", ctypes.c_uint64), ("repeated", ctypes.c_uint64), ("yielded", ctypes.c_uint64)]
 
 
 # Names of the array members and their (dtype, per-item width, count key).

@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <fstream>
 #include <string>
 #include <thread>
@@ -907,8 +908,9 @@ static int darcy_correct(sph_ctx *ctx, const DarcyArgs &da, double *pc)
 // each learned correction (after sweeps 1, 11, 21, ...), then one to the end.
 // The launches alternate between the two iterate buffers; out is the one that
 // holds the solve's result, h_state the solve state.  With resident = false
-// on return a wait ran out: the solve is back at its start, and this context
-// goes on with one launch per sweep.
+// on return the solve is back at its start: a wait ran out, and this context
+// goes on with one launch per sweep, or the solve yields to grid barriers
+// (resident_begin) and takes one launch per sweep itself.
 static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2], bool &resident, int &out)
 {
     const sph_state &h = ctx->hs.h;
@@ -924,9 +926,13 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
         const unsigned int end = it + std::min(len, h.maxiter - it);
         ResidentArgs a;
         bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->res_wait, a);
+        bool yields = false;
         if (ok) {
             ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
-            launch_darcy_resident(s, ctx->device, ctx->res, a, da, d, buf[cur], buf[cur ^ 1], h.tolerance);
+            yields = !launch_darcy_resident(s, ctx->device, ctx->res, a, da, d, buf[cur], buf[cur ^ 1], h.tolerance);
+            ok = !yields;
+        }
+        if (ok) {
             cur ^= 1;
             ends.push_back(end);
             if (learned && end % 10u == 2u) {
@@ -943,8 +949,12 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
         const int rc = sync(ctx);
         if (rc) return rc;
         if (!ok || ctx->h_state[0] == RES_ABORT) {
-            if (ctx->h_state[0] == RES_ABORT) ctx->res.repeated++;
-            ctx->res.usable = false;
+            if (yields) {
+                ctx->res.yielded++;
+            } else {
+                ctx->res.repeated += ctx->h_state[0] == RES_ABORT;
+                ctx->res.usable = false;
+            }
             resident = false;
             launch_darcy_copy_interior(s, da, d.p_old, buf[0]);
             launch_darcy_ghosts(s, da, buf[0], 1);
@@ -1368,6 +1378,13 @@ static bool gather_in_integrate(const sph_ctx *ctx)
     return !h.fluid && !ctx->ns && !(h.nw > 0 && h.wmode[0] == 3);
 }
 
+// The context's steps run grid barriers (launch_rebuild): their callers hold a
+// BarrierUse.
+static bool runs_barriers(const sph_ctx *ctx)
+{
+    return ctx->nl_on && ctx->rb_blocks && !ctx->hs.h.fluid && !ctx->ns;
+}
+
 static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *dir,
                      const std::string &sid)
 {
@@ -1403,7 +1420,7 @@ static int step_once(sph_ctx *ctx, std::ofstream *convlog, const std::string *di
                 std::swap(ctx->db.vals, ctx->db.vals_tmp);
             }
             ctx->hash_aside = false;
-            if (ctx->rb_blocks && !fluid) {
+            if (runs_barriers(ctx)) {
                 ProfScope ps(ctx, SPH_K_NLIST);
                 launch_rebuild(s, a, ctx->nla, ctx->db, ctx->ncells, ctx->key_bits,
                                ctx->rb_blocks, cond, ctx->rb_spin);
@@ -1660,7 +1677,7 @@ int sph_set_resident_wait_limit(sph_ctx *ctx, uint32_t polls, uint32_t from_swee
 int sph_get_resident_stats(sph_ctx *ctx, sph_resident_stats *out)
 {
     if (!ctx || !out) return fail(ctx, SPH_ERR_ARG, "null argument");
-    *out = sph_resident_stats{ctx->res.solves, ctx->res.repeated};
+    *out = sph_resident_stats{ctx->res.solves, ctx->res.repeated, ctx->res.yielded};
     return SPH_OK;
 }
 
@@ -1794,6 +1811,8 @@ int sph_step(sph_ctx *ctx, int nsteps)
     if (!ctx) return fail(ctx, SPH_ERR_ARG, "null context");
     if (!ctx->loaded) return fail(ctx, SPH_ERR_STATE, "no state loaded");
     (void)hipSetDevice(ctx->device);
+    BarrierUse barriers;
+    if (runs_barriers(ctx)) barriers.open(ctx->device, ctx->stream);
     for (int i = 0; i < nsteps; ++i) {
         int rc = step_once(ctx, nullptr, nullptr, std::string());
         if (rc) return rc;
@@ -1866,6 +1885,8 @@ int sph_run(const sph_run_opts *opts)
     }
     std::ofstream convlog((dir + "/" + sid + "-conv.log").c_str());
     long nstep = 0;
+    BarrierUse barriers;
+    if (runs_barriers(ctx)) barriers.open(ctx->device, ctx->stream);
     while (h.time_current <= h.time_total) {
         rc = step_once(ctx, &convlog, &dir, sid);
         if (!rc && (++nstep % 64 == 0)) rc = check_flags(ctx);
@@ -1879,6 +1900,7 @@ int sph_run(const sph_run_opts *opts)
     if (!rc) rc = sync(ctx);
     if (opts->verbose) printf("\n");
     if (rc) g_last_error = ctx->err;
+    barriers.close();
     sph_destroy(ctx);
     return rc;
 }
@@ -2536,6 +2558,8 @@ int sph_ensemble_autotune(sph_ensemble *e, int trial_steps, const double *fracti
     for (size_t k = 0; k < e->boxes.size(); ++k) {
         sph_ctx *c = e->boxes[k];
         double best = 1e300, best_f = c->nl_frac;
+        BarrierUse barriers;
+        if (runs_barriers(c)) barriers.open(c->device, c->stream);
         const bool tunable = c->loaded && c->nl_on;
         for (int f = 0; f < nfrac; ++f) {
             double ms = -1.0;
@@ -3084,15 +3108,18 @@ int sph_ensemble_step(sph_ensemble *e, int nsteps)
         if ((rc = sync(c))) return ens_fail(e, rc, c->err);
     if (!ens_plan_current(e) && (rc = ens_plan(e))) return rc;
     if (!ens_fluid_current(e) && (rc = ens_fluid_plan(e))) return rc;
-    std::vector<sph_ctx *> single;
+    std::vector<sph_ctx *> single, single_fluid;
     {
         size_t i = 0, f = 0;
         for (size_t k = 0; k < e->boxes.size(); ++k) {
+            sph_ctx *c = e->boxes[k];
             if (i < e->multi.size() && e->multi[i] == (int)k) ++i;
             else if (f < e->fluid.size() && e->fluid[f] == (int)k) ++f;
-            else single.push_back(e->boxes[k]);
+            else (c->hs.h.fluid || c->ns ? single_fluid : single).push_back(c);
         }
     }
+    BarrierUse barriers;
+    if (!e->multi.empty() || !e->fluid.empty()) barriers.open(e->device, e->stream);
     int left = nsteps;
     if (!e->multi.empty()) {
         // the hash of a box's first step after a load (later ones are
@@ -3147,8 +3174,19 @@ int sph_ensemble_step(sph_ensemble *e, int nsteps)
         for (int k = 0; k < nsteps; ++k)
             if ((rc = ens_fluid_step(e))) return rc;
     // the other boxes, box by box on their own streams
+    {
+        std::deque<BarrierUse> own(single.size());
+        for (size_t i = 0; i < single.size(); ++i)
+            if (runs_barriers(single[i])) own[i].open(e->device, single[i]->stream);
+        for (int k = 0; k < nsteps; ++k)
+            for (sph_ctx *c : single)
+                if ((rc = step_once(c, nullptr, nullptr, std::string()))) return ens_fail(e, rc, c->err);
+    }
+    // the fluids among them once no grid barrier is in flight, so that their
+    // sweeps are resident (resident.h)
+    if (!single_fluid.empty()) barriers.close();
     for (int k = 0; k < nsteps; ++k)
-        for (sph_ctx *c : single)
+        for (sph_ctx *c : single_fluid)
             if ((rc = step_once(c, nullptr, nullptr, std::string()))) return ens_fail(e, rc, c->err);
     HIPCHK_E(hipStreamSynchronize(e->stream));
     for (sph_ctx *c : e->boxes) {

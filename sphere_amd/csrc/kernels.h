@@ -351,7 +351,8 @@ void launch_darcy_sweep(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b
                         bool zero_scale = false);
 // sweeps in one resident launch (resident.h), where the boundaries allow it
 bool darcy_resident_form(const DarcyArgs &d, int &wrap);
-void launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
+// (false: not now, resident_begin)
+bool launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
                            const DarcyArgs &d, const DarcyBuffers &b, const double *p_in, double *p_out,
                            double tolerance);
 void launch_darcy_residual_max(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b, const double *p,

@@ -887,9 +887,10 @@ int read_state(sph_ns *n)
 }
 
 // The Jacobi iterations of a solve in resident launches, each from
-// eps[cur] into the other buffer.  With resident = false on return a wait
-// ran out: the iterate is back at the solve's start, and this fluid goes on
-// with one launch per iteration.
+// eps[cur] into the other buffer.  With resident = false on return the iterate
+// is back at the solve's start: a wait ran out, and this fluid goes on with one
+// launch per iteration, or the solve yields to grid barriers (resident_begin)
+// and takes one launch per iteration itself.
 int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
 {
     const sph_ns_params &P = n->P;
@@ -916,20 +917,25 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
         ResidentArgs a;
         bool ok = resident_args(n->res, n->s, g.nx, g.ny, g.nz, it, it + std::min(chunk, P.maxiter - it),
                                 n->res_wait, a);
+        bool yields = false;
         if (ok) {
             const NsOp op{g, n->q, n->eps[n->cur], n->eps[1 - n->cur], cv(n->vp), cv(n->vpf), n->phi, n->dphi,
                           n->dst, P.tolerance, n->dp_dz, n->wall0_iz, fixed_div(2.0 * g.dx),
                           fixed_div(2.0 * g.dy), fixed_div(2.0 * g.dz),
                           fixed_div(2.0 * (dxdx * dydy + dxdx * dzdz + dydy * dzdz))};
-            resident_launch(n->res, n->device, n->s, a, op);
+            yields = !resident_launch(n->res, n->device, n->s, a, op);
             rc = hip_ok(hipGetLastError(), "Navier-Stokes resident iterations");
-            if (!rc) rc = read_state(n);
+            if (!rc && !yields) rc = read_state(n);
             if (rc) return rc;
-            ok = n->hst->done != RES_ABORT;
+            ok = !yields && n->hst->done != RES_ABORT;
         }
         if (!ok) {
-            if (n->hst->done == RES_ABORT) n->res.repeated++;
-            n->res.usable = false;
+            if (yields) {
+                n->res.yielded++;
+            } else {
+                n->res.repeated += n->hst->done == RES_ABORT;
+                n->res.usable = false;
+            }
             resident = false;
             n->cur = cur0;
             rc = hip_ok(hipMemsetAsync(n->dst, 0, sizeof(NsSolveState), n->s), "hipMemsetAsync");
@@ -1451,7 +1457,7 @@ int sph_ns_get_stats(const sph_ns *n, sph_ns_stats *out)
 int sph_ns_get_resident_stats(const sph_ns *n, sph_resident_stats *out)
 {
     if (!n || !out) return fail(SPH_ERR_ARG, "bad argument");
-    *out = sph_resident_stats{n->res.solves, n->res.repeated};
+    *out = sph_resident_stats{n->res.solves, n->res.repeated, n->res.yielded};
     return SPH_OK;
 }
 

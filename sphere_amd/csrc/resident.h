@@ -30,7 +30,15 @@
 // with one launch per sweep.  Blocks of one launch need to be resident
 // together: the grid is at most one block per compute unit, and
 // resident_begin() and resident_end() let the resident launches of a device
-// follow each other.
+// follow each other.  The grid barriers of the list rebuild (k_rebuild,
+// k_rebuild_lists, k_rebuild_multi) need the same of their blocks, and a compute
+// unit that holds a block of 1024 threads at 104 registers has room for one
+// block of theirs: partly placed, the two kinds could keep each other's rest
+// out until a bound runs out.  So both are never in flight together: a call
+// that may enqueue rebuilds holds a BarrierUse, whose stream waits for the last
+// resident launch, and while one is held elsewhere a solve takes one launch
+// per sweep.  Another process on the card is not seen: there the bound ends
+// the wait.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -76,6 +84,7 @@ struct Resident {
     bool planned = false;
     uint64_t solves = 0;                  // solves whose result came from resident launches
     uint64_t repeated = 0;                // solves in which a wait ran out
+    uint64_t yielded = 0;                 // solves left to launches per sweep by a BarrierUse
 };
 // The bound of the waits of the launches that begin at iteration `from` or
 // later, in polls (0: RES_SPIN, as for the others).
@@ -91,9 +100,24 @@ void resident_free(Resident &r);
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,
                    const ResidentWait &wait, ResidentArgs &out);
 // Resident launches of one device wait for each other: call before and after
-// the launch.
-void resident_begin(int device, hipStream_t s);
+// the launch.  False, and then no launch: a BarrierUse of the device is held.
+bool resident_begin(int device, hipStream_t s);
 void resident_end(int device, hipStream_t s);
+
+// Held while stream s of a device may run grid barriers.
+class BarrierUse {
+public:
+    BarrierUse() = default;
+    BarrierUse(const BarrierUse &) = delete;
+    BarrierUse &operator=(const BarrierUse &) = delete;
+    ~BarrierUse() { close(); }
+    void open(int device, hipStream_t s);
+    void close();  // waits for the stream first
+
+private:
+    int device_ = -1;
+    hipStream_t stream_ = nullptr;
+};
 
 #if defined(__HIPCC__)
 
@@ -429,15 +453,17 @@ __global__ void __launch_bounds__(1024) k_resident_jacobi(ResidentArgs r, Op op)
     }
 }
 
+// false: not now (resident_begin)
 template <class Op>
-void resident_launch(const Resident &r, int device, hipStream_t s, const ResidentArgs &a, const Op &op)
+bool resident_launch(const Resident &r, int device, hipStream_t s, const ResidentArgs &a, const Op &op)
 {
-    resident_begin(device, s);
+    if (!resident_begin(device, s)) return false;
     if (r.per_thread == 1)
         hipLaunchKernelGGL((k_resident_jacobi<Op, 1>), dim3(r.tiles), dim3(r.threads), r.lds, s, a, op);
     else
         hipLaunchKernelGGL((k_resident_jacobi<Op, 2>), dim3(r.tiles), dim3(r.threads), r.lds, s, a, op);
     resident_end(device, s);
+    return true;
 }
 
 #endif

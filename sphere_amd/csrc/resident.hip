@@ -1,6 +1,6 @@
 // resident.hip -- host side of the resident Jacobi launches (resident.h):
-// the division of a cell grid into tiles, the outboxes, and the order of the
-// resident launches of a device.
+// the division of a cell grid into tiles, the outboxes, and the order of a
+// device's resident launches and grid barriers.
 #include "resident.h"
 
 #include <algorithm>
@@ -12,6 +12,7 @@ struct DeviceOrder {
     std::mutex m;
     hipEvent_t last = nullptr;
     bool any = false;
+    uint32_t barriers = 0;  // BarrierUses held
 };
 constexpr int MAX_DEVICES = 64;
 DeviceOrder g_order[MAX_DEVICES];
@@ -108,11 +109,16 @@ bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t 
     return true;
 }
 
-void resident_begin(int device, hipStream_t s)
+bool resident_begin(int device, hipStream_t s)
 {
     DeviceOrder &o = g_order[device];
     o.m.lock();
+    if (o.barriers) {
+        o.m.unlock();
+        return false;
+    }
     if (o.any) (void)hipStreamWaitEvent(s, o.last, 0);
+    return true;
 }
 
 void resident_end(int device, hipStream_t s)
@@ -121,4 +127,26 @@ void resident_end(int device, hipStream_t s)
     if (!o.last && hipEventCreateWithFlags(&o.last, hipEventDisableTiming) != hipSuccess) o.last = nullptr;
     o.any = o.last && hipEventRecord(o.last, s) == hipSuccess;
     o.m.unlock();
+}
+
+void BarrierUse::open(int device, hipStream_t s)
+{
+    close();
+    if (device < 0 || device >= MAX_DEVICES) return;  // no resident launches there
+    DeviceOrder &o = g_order[device];
+    std::lock_guard<std::mutex> lock(o.m);
+    ++o.barriers;
+    if (o.any) (void)hipStreamWaitEvent(s, o.last, 0);
+    device_ = device;
+    stream_ = s;
+}
+
+void BarrierUse::close()
+{
+    if (device_ < 0) return;
+    (void)hipStreamSynchronize(stream_);
+    DeviceOrder &o = g_order[device_];
+    std::lock_guard<std::mutex> lock(o.m);
+    --o.barriers;
+    device_ = -1;
 }
