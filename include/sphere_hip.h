@@ -218,9 +218,10 @@ int sph_set_barrier_spin_limit(sph_ctx *ctx, uint32_t sleeps);
  * the reference.  The limit bounds those waits, in polls, for the launches that
  * begin at sweep from_sweep of a solve or later (0: the default, 2^20, about a
  * second).  Where a wait runs out, the solve is repeated with one launch per
- * sweep, to the same bits, as are the later ones.  A small bound forces that
- * path from the host.  It holds for the context's Darcy fluid and for an
- * attached Navier-Stokes fluid; takes effect at once. */
+ * sweep, to the same bits, as are the next 16 solves, twice as many after each
+ * further such wait.  A small bound forces that path from the host.  It holds
+ * for the context's Darcy fluid and for an attached Navier-Stokes fluid; takes
+ * effect at once. */
 int sph_set_resident_wait_limit(sph_ctx *ctx, uint32_t polls, uint32_t from_sweep);
 
 /* How the solves of the loaded state's Darcy fluid ran (sph_ns_get_resident_stats:

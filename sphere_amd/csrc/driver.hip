@@ -908,9 +908,9 @@ static int darcy_correct(sph_ctx *ctx, const DarcyArgs &da, double *pc)
 // each learned correction (after sweeps 1, 11, 21, ...), then one to the end.
 // The launches alternate between the two iterate buffers; out is the one that
 // holds the solve's result, h_state the solve state.  With resident = false
-// on return the solve is back at its start: a wait ran out, and this context
-// goes on with one launch per sweep, or the solve yields to grid barriers
-// (resident_begin) and takes one launch per sweep itself.
+// on return the solve is back at its start, and takes one launch per sweep: a
+// wait ran out (resident_gave_up), or the solve yields to grid barriers
+// (resident_begin).
 static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2], bool &resident, int &out)
 {
     const sph_state &h = ctx->hs.h;
@@ -949,12 +949,9 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
         const int rc = sync(ctx);
         if (rc) return rc;
         if (!ok || ctx->h_state[0] == RES_ABORT) {
-            if (yields) {
-                ctx->res.yielded++;
-            } else {
-                ctx->res.repeated += ctx->h_state[0] == RES_ABORT;
-                ctx->res.usable = false;
-            }
+            if (yields) ctx->res.yielded++;
+            else if (ctx->h_state[0] == RES_ABORT) resident_gave_up(ctx->res);
+            else ctx->res.usable = false;
             resident = false;
             launch_darcy_copy_interior(s, da, d.p_old, buf[0]);
             launch_darcy_ghosts(s, da, buf[0], 1);
@@ -1033,7 +1030,7 @@ static int darcy_step(sph_ctx *ctx, std::ofstream *convlog)
     bool resident = darcy_resident_form(da, wrap);
     if (resident && !ctx->res.planned)
         resident_plan(ctx->res, ctx->device, (int)da.nx, (int)da.ny, (int)da.nz, wrap);
-    resident = resident && ctx->res.usable;
+    resident = resident && resident_ready(ctx->res);
     if (resident) {
         rc0 = darcy_resident(ctx, da, buf, resident, out);
         if (rc0) return rc0;

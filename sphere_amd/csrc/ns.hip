@@ -888,9 +888,8 @@ int read_state(sph_ns *n)
 
 // The Jacobi iterations of a solve in resident launches, each from
 // eps[cur] into the other buffer.  With resident = false on return the iterate
-// is back at the solve's start: a wait ran out, and this fluid goes on with one
-// launch per iteration, or the solve yields to grid barriers (resident_begin)
-// and takes one launch per iteration itself.
+// is back at the solve's start, and takes one launch per iteration: a wait ran
+// out (resident_gave_up), or the solve yields to grid barriers (resident_begin).
 int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
 {
     const sph_ns_params &P = n->P;
@@ -930,12 +929,9 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
             ok = !yields && n->hst->done != RES_ABORT;
         }
         if (!ok) {
-            if (yields) {
-                n->res.yielded++;
-            } else {
-                n->res.repeated += n->hst->done == RES_ABORT;
-                n->res.usable = false;
-            }
+            if (yields) n->res.yielded++;
+            else if (n->hst->done == RES_ABORT) resident_gave_up(n->res);
+            else n->res.usable = false;
             resident = false;
             n->cur = cur0;
             rc = hip_ok(hipMemsetAsync(n->dst, 0, sizeof(NsSolveState), n->s), "hipMemsetAsync");
@@ -1013,7 +1009,7 @@ int ns_solve(sph_ns *n)
     // not) keeps a different value in each buffer: one launch per iteration
     if (!n->res.planned)
         resident_plan(n->res, n->device, g.nx, g.ny, g.nz, 3 | (g.bb == 2 && g.bt == 2 ? 4 : 0));
-    bool resident = n->res.usable && (g.bb == 2) == (g.bt == 2);
+    bool resident = (g.bb == 2) == (g.bt == 2) && resident_ready(n->res);
     if (resident) {
         rc = ns_resident(n, resident, converged, nijac);
         if (rc) return rc;

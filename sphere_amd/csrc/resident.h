@@ -82,6 +82,8 @@ struct Resident {
     uint32_t tag = 1;                     // next unused tag
     bool usable = false;                  // false: one launch per sweep
     bool planned = false;
+    uint32_t rest = 0;                    // solves left to launches per sweep after a wait ran out
+    uint32_t pause = 0;                   // their number after the last such wait
     uint64_t solves = 0;                  // solves whose result came from resident launches
     uint64_t repeated = 0;                // solves in which a wait ran out
     uint64_t yielded = 0;                 // solves left to launches per sweep by a BarrierUse
@@ -95,6 +97,12 @@ struct ResidentWait {
 // where the grid does not fit (see resident.hip).
 void resident_plan(Resident &r, int device, int nx, int ny, int nz, int wrap);
 void resident_free(Resident &r);
+// The next solve is to run in resident launches.
+bool resident_ready(Resident &r);
+// A wait ran out: the next 16 solves, and twice as many after each further such
+// wait, are left to launches per sweep (what kept a block out, another process
+// on the card for instance, may have gone by then, and a wait costs a second).
+void resident_gave_up(Resident &r);
 // The arguments of one launch over iterations [it0, it1); false if the outboxes
 // could not be made.
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,

@@ -76,6 +76,21 @@ void resident_free(Resident &r)
     r = Resident{};
 }
 
+bool resident_ready(Resident &r)
+{
+    if (!r.usable) return false;
+    if (r.rest == 0) return true;
+    --r.rest;
+    return false;
+}
+
+void resident_gave_up(Resident &r)
+{
+    r.repeated++;
+    r.pause = r.pause ? std::min(2u * r.pause, 65536u) : 16u;
+    r.rest = r.pause;
+}
+
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,
                    const ResidentWait &wait, ResidentArgs &out)
 {

@@ -83,6 +83,28 @@ def test_wait_bound_falls_back():
         assert numpy.array_equal(got[0][0][k], got[1][0][k]), k
 
 
+def test_resident_again_after_a_pause():
+    """After a wait has run out 16 solves, then 32, take one launch per sweep,
+    and the next one is resident again."""
+    s = darcy_case(n=200, seed=3, nxyz=(5, 9, 8), tolerance=1e-7)
+    ref, e = sphere_amd.Engine(0), sphere_amd.Engine(0)
+    ref.load(s.to_state())
+    e.load(s.to_state())
+    for polls, steps, want in ((1, 17, (0, 1)), (1, 1, (0, 2)), (0, 32, (0, 2)), (0, 2, (2, 2))):
+        e.set_resident_wait_limit(polls)
+        print("darcy, wait bound", polls, steps, "steps", flush=True)
+        e.step(steps)
+        rs = e.resident_stats()
+        assert (rs.solves, rs.repeated) == want
+    ref.step(52)
+    assert ref.resident_stats().solves == 52 and ref.darcy_stats().sweeps == e.darcy_stats().sweeps
+    a, b = e.read().arrays, ref.read().arrays
+    for k in ("p_f", "x", "vel", "force"):
+        assert numpy.array_equal(a[k], b[k]), k
+    e.close()
+    ref.close()
+
+
 @pytest.mark.parametrize("learned,later", [(True, 2), (True, 12), (True, 22), (False, 20000)])
 def test_wait_bound_in_a_later_launch(learned, later):
     """A wait that runs out after earlier launches of the solve have written
