@@ -245,6 +245,10 @@ int sph_get_header(sph_ctx *ctx, sph_state *hdr);
 /* Copy the device state into caller buffers (any NULL array is skipped):
  * replaces transferFromGlobalDeviceMemory (src/device.cu:754-829). */
 int sph_read_state(sph_ctx *ctx, sph_state *out);
+/* The copy goes through pinned staging memory that the contexts of a process
+ * share (on = 1, the default), or straight to the caller's buffers (on = 0, and
+ * where no pinned memory can be had). */
+int sph_set_read_staging(sph_ctx *ctx, int on);
 /* Write the current state as a v2.15 file: replaces DEM::writebin
  * (src/file_io.cpp:420-731). */
 int sph_write_file(sph_ctx *ctx, const char *path);

@@ -206,6 +206,7 @@ def load_library(path=None):
         "sph_set_rebuild_kernel": (ctypes.c_int, [vp, ctypes.c_int]),
         "sph_set_barrier_spin_limit": (ctypes.c_int, [vp, ctypes.c_uint32]),
         "sph_set_resident_wait_limit": (ctypes.c_int, [vp, ctypes.c_uint32, ctypes.c_uint32]),
+        "sph_set_read_staging": (ctypes.c_int, [vp, ctypes.c_int]),
         "sph_get_resident_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphResidentStats)]),
         "sph_get_neighbor_stats": (ctypes.c_int, [vp, ctypes.POINTER(SphNeighborStats)]),
         "sph_load_state": (ctypes.c_int, [vp, ctypes.POINTER(SphState)]),
@@ -399,6 +400,11 @@ class Engine:
         s = SphNeighborStats()
         self._check(self.lib.sph_get_neighbor_stats(self.ctx, ctypes.byref(s)))
         return s
+
+    def set_read_staging(self, on):
+        """State reads through pinned staging memory (the default), or straight
+        to the destination."""
+        self._check(self.lib.sph_set_read_staging(self.ctx, int(on)))
 
     def set_barrier_spin_limit(self, sleeps):
         """Bound of the list rebuild kernel's grid-barrier waits and of the

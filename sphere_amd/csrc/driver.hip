@@ -19,6 +19,7 @@
 #include <cstring>
 #include <deque>
 #include <fstream>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <tuple>
@@ -96,9 +97,7 @@ struct sph_ctx {
     int net_max_corr = 0;
     sph_net *net = nullptr;
     float *net_params = nullptr, *net_in = nullptr, *net_out = nullptr;
-    // pinned staging of state reads (read_rows), made at the first read
-    char *read_pin = nullptr;
-    size_t read_cap = 0;
+    bool read_staging = true;  // state reads through pinned memory (read_rows)
     // profiling
     bool prof = false;
     double ktime[SPH_K_COUNT] = {0};
@@ -257,9 +256,6 @@ static void free_device(sph_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     ctx->end_pending = false;
     resident_free(ctx->res);
-    if (ctx->read_pin) (void)hipHostFree(ctx->read_pin);
-    ctx->read_pin = nullptr;
-    ctx->read_cap = 0;
     for (void *p : ctx->allocs) (void)hipFree(p);
     ctx->allocs.clear();
     ctx->db = DemBuffers{};
@@ -631,16 +627,84 @@ struct ReadRow {
     size_t bytes;
 };
 
-// Copies the rows through pinned memory.  hipMemcpy into pageable memory
-// moved a 1,000,000-grain state at 7 GB/s (30 ms), because one thread copies
+// Pinned staging memory of the state reads, one pool for all contexts: a read
+// takes a piece and gives it back, so that a set of boxes read one after another
+// makes one piece, not one per box and load: loading and reading 16 boxes of
+// 1,000 to 30,000 grains again takes 21.9 ms, 26.3 with a piece per context and
+// load, 23.4 with hipMemcpy straight to the destinations.  At most PINNED_IDLE
+// pieces of up to 16 MB wait in it, and none once the last context is destroyed.
+#define PINNED_IDLE 4u
+struct Pinned {
+    char *p = nullptr;
+    size_t bytes = 0;
+};
+class PinnedPool {
+public:
+    void enter()
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        ++contexts_;
+    }
+    void leave()
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        if (--contexts_ == 0)
+            while (!idle_.empty()) drop(idle_.size() - 1);
+    }
+    // the smallest piece that holds `bytes`, else a new one of the next power of
+    // two; p is null where none can be made
+    Pinned take(size_t bytes)
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        size_t best = idle_.size();
+        for (size_t k = 0; k < idle_.size(); ++k)
+            if (idle_[k].bytes >= bytes && (best == idle_.size() || idle_[k].bytes < idle_[best].bytes)) best = k;
+        Pinned q;
+        if (best < idle_.size()) {
+            q = idle_[best];
+            idle_.erase(idle_.begin() + (long)best);
+            return q;
+        }
+        for (q.bytes = size_t(256) << 10; q.bytes < bytes;) q.bytes *= 2;
+        if (hipHostMalloc((void **)&q.p, q.bytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            q.p = nullptr;
+        }
+        return q;
+    }
+    void give(const Pinned &q)
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        idle_.push_back(q);
+        if (idle_.size() <= PINNED_IDLE) return;
+        size_t least = 0;
+        for (size_t k = 1; k < idle_.size(); ++k)
+            if (idle_[k].bytes < idle_[least].bytes) least = k;
+        drop(least);
+    }
+
+private:
+    void drop(size_t k)
+    {
+        (void)hipHostFree(idle_[k].p);
+        idle_.erase(idle_.begin() + (long)k);
+    }
+    std::mutex m_;
+    std::vector<Pinned> idle_;
+    size_t contexts_ = 0;
+};
+static PinnedPool g_pinned;
+
+// Copies the rows through pinned memory, or straight to their destinations
+// where there is none.  hipMemcpy into pageable memory moved a 1,000,000-grain state at 7 GB/s (30 ms), because one thread copies
 // out of the driver's staging buffer and takes the page faults of a
 // destination that has not been touched.  Here READ_THREADS threads move
 // pieces, each through a staging piece of its own.  A state
 // that fits into the staging memory at once, up to READ_SMALL, is copied with
 // one wait and no threads (0.6 ms for 1,000 grains with a wait per array).
 #define READ_THREADS 8
-// A piece is 1/32 of the state, 512 KB to 2 MB: 2 MB ones take each of many
-// small boxes 1 ms to make, 512 KB ones cost a 224 MB state 4 ms per read.
+// A thread's piece is 1/32 of the state, 512 KB to 2 MB: 512 KB ones cost a
+// 224 MB state 4 ms per read, 2 MB ones a 4 MB state 1 ms to make.
 #define READ_PIECE_MIN (size_t(512) << 10)
 #define READ_PIECE_MAX (size_t(2) << 20)
 #define READ_SMALL (size_t(4) << 20)
@@ -651,24 +715,31 @@ static int read_rows(sph_ctx *ctx, const std::vector<ReadRow> &rows)
     if (!total) return SPH_OK;
     const bool small = total <= READ_SMALL;
     const size_t piece = std::min(READ_PIECE_MAX, std::max(READ_PIECE_MIN, total / 32 / 4096 * 4096));
-    const size_t cap = small ? total : READ_THREADS * piece;
-    if (ctx->read_cap < cap) {
-        if (ctx->read_pin) (void)hipHostFree(ctx->read_pin);
-        ctx->read_pin = nullptr;
-        ctx->read_cap = 0;
-        HIPCHK(hipHostMalloc((void **)&ctx->read_pin, cap, hipHostMallocDefault));
-        ctx->read_cap = cap;
+    struct Staging {  // given back once no copy into it is in flight
+        hipStream_t s;
+        Pinned q;
+        ~Staging()
+        {
+            if (!q.p) return;
+            (void)hipStreamSynchronize(s);
+            g_pinned.give(q);
+        }
+    } staging{ctx->stream, ctx->read_staging ? g_pinned.take(small ? total : READ_THREADS * piece) : Pinned{}};
+    char *const pinned = staging.q.p;
+    if (!pinned) {
+        for (const ReadRow &r : rows) HIPCHK(hipMemcpy(r.dst, r.src, r.bytes, hipMemcpyDeviceToHost));
+        return SPH_OK;
     }
     if (small) {
         size_t at = 0;
         for (const ReadRow &r : rows) {
-            HIPCHK(hipMemcpyAsync(ctx->read_pin + at, r.src, r.bytes, hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(hipMemcpyAsync(pinned + at, r.src, r.bytes, hipMemcpyDeviceToHost, ctx->stream));
             at += (r.bytes + 255) / 256 * 256;
         }
         HIPCHK(hipStreamSynchronize(ctx->stream));
         at = 0;
         for (const ReadRow &r : rows) {
-            std::memcpy(r.dst, ctx->read_pin + at, r.bytes);
+            std::memcpy(r.dst, pinned + at, r.bytes);
             at += (r.bytes + 255) / 256 * 256;
         }
         return SPH_OK;
@@ -683,7 +754,7 @@ static int read_rows(sph_ctx *ctx, const std::vector<ReadRow> &rows)
     auto work = [&](int t) {
         hipError_t e = err[t];
         if (e == hipSuccess) e = hipSetDevice(ctx->device);
-        char *pin = ctx->read_pin + (size_t)t * piece;
+        char *pin = pinned + (size_t)t * piece;
         for (size_t k = (size_t)t; k < pieces.size() && e == hipSuccess; k += READ_THREADS) {
             e = hipMemcpyAsync(pin, pieces[k].src, pieces[k].bytes, hipMemcpyDeviceToHost, ctx->stream);
             if (e == hipSuccess) e = hipEventRecord(ev[t], ctx->stream);
@@ -1545,6 +1616,7 @@ sph_ctx *sph_create(int device)
         delete ctx;
         return nullptr;
     }
+    g_pinned.enter();
     ctx->h_u64 = (unsigned long long *)((char *)ctx->h_err + 16);
     ctx->h_d = (double *)((char *)ctx->h_err + 32);
     ctx->h_state = (unsigned long long *)((char *)ctx->h_err + 64);
@@ -1586,6 +1658,7 @@ void sph_destroy(sph_ctx *ctx)
     if (ctx->h_err) (void)hipHostFree(ctx->h_err);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
+    g_pinned.leave();
 }
 
 const char *sph_last_error(const sph_ctx *ctx)
@@ -1752,6 +1825,13 @@ int sph_get_header(sph_ctx *ctx, sph_state *hdr)
     hdr->v_f = hdr->p_f = hdr->phi = hdr->dphi = hdr->f_p = nullptr;
     hdr->p_constant = nullptr;
     hdr->color = nullptr;
+    return SPH_OK;
+}
+
+int sph_set_read_staging(sph_ctx *ctx, int on)
+{
+    if (!ctx) return fail(ctx, SPH_ERR_ARG, "null context");
+    ctx->read_staging = on != 0;
     return SPH_OK;
 }
 
