@@ -2218,8 +2218,9 @@ int sph_kernel_time(sph_ctx *ctx, int kernel_id, double *total_ms, uint64_t *lau
 // (the rebuild-flag word and, for an odd number of radix passes, which key
 // buffer is current), so a plan holds the records of two consecutive
 // steps, and two steps are captured in one HIP graph that is replayed.
-// Other boxes (fluid, cell search, shear-stress walls, ...) are stepped
-// box by box on their own streams beside the multi-box launches.
+// Other boxes (cell search, shear-stress walls, ...) are stepped box by box on
+// their own streams beside the multi-box launches, those with a fluid that is
+// not stepped together (below) after them.
 // ------------------------------------------------------------------
 
 }  // extern "C"
@@ -2313,12 +2314,12 @@ static void ens_drop_plan(sph_ensemble *e)
 }
 
 // A box the multi-box launches can step: the list path with the fused
-// rebuild, contact model 2 or 3, no fluid, no adaptive grid, no wmode-3
-// wall, no profiling.
+// rebuild, contact model 2 or 3, no fluid (its own or attached), no adaptive
+// grid, no wmode-3 wall, no profiling.
 static bool ens_multi_eligible(const sph_ctx *c)
 {
     const sph_state &h = c->hs.h;
-    return c->loaded && h.np > 0 && !h.fluid && c->nl_on && c->rb_cap > 0 &&
+    return c->loaded && h.np > 0 && !h.fluid && !c->ns && c->nl_on && c->rb_cap > 0 &&
            (h.contactmodel == 2 || h.contactmodel == 3) && !(h.adaptive == 1 && h.nw > 0) &&
            !(h.nw > 0 && h.wmode[0] == 3) && !c->prof && c->db.rb_bar && c->db.rb_part;
 }
