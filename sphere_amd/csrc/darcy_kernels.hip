@@ -983,11 +983,11 @@ bool darcy_resident_form(const DarcyArgs &d, int &wrap)
 // verdicts go into the solve state like those of the single sweeps.
 bool launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
                            const DarcyArgs &d, const DarcyBuffers &b, const double *p_in, double *p_out,
-                           double tolerance)
+                           double tolerance, uint32_t held)
 {
     const DarcyOp op{d, b.jc, b.jfrozen, p_in, p_out, b.maxres + DARCY_STATE, b.maxres + DARCY_SCALE, tolerance,
                      fixed_div(d.dx), fixed_div(d.dy), fixed_div(d.dz)};
-    return resident_launch(r, device, s, a, op);
+    return resident_launch(r, device, s, a, op, held);
 }
 
 // The test of a check sweep that no sweep follows (the last of maxiter).

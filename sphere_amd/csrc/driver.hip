@@ -975,6 +975,62 @@ static int darcy_correct(sph_ctx *ctx, const DarcyArgs &da, double *pc)
     return SPH_OK;
 }
 
+// Sweeps [from, maxiter) of a solve with one launch each, on stream s, until the
+// solve has ended; sweep n reads buf[n & 1] and writes the other.  The
+// convergence test of check sweep j (j % 10 == 0) runs on the device at the
+// start of sweep j + 1, and once it ends the solve every later sweep returns at
+// once.  The host enqueues sweeps in batches (the first as long as the last
+// solve, each ending with a deciding sweep) and reads the solve state into
+// h_state once per batch.
+static int darcy_launches(sph_ctx *ctx, hipStream_t s, const DarcyArgs &da, double *const buf[2],
+                          unsigned int from, int corrections)
+{
+    const sph_state &h = ctx->hs.h;
+    const DarcyBuffers &d = ctx->dd;
+    unsigned int nijac = from;
+    unsigned long long want = std::max(from / 10u * 10u + 12u, (ctx->jacobi_hint + 9u) / 10u * 10u + 2u);
+    std::memset(ctx->h_state, 0, 32);
+    while (nijac < h.maxiter && ctx->h_state[0] == 0) {
+        const unsigned int end = (unsigned int)std::min<unsigned long long>(h.maxiter, want);
+        for (; nijac < end; ++nijac) {
+            const bool check = (nijac % 10 == 0);
+            // two check slots alternate: a check sweep zeroes the other one
+            unsigned long long *slot = d.maxres + ((nijac / 10) & 1u) * RED_WORDS;
+            unsigned long long *next = d.maxres + (((nijac / 10) & 1u) ^ 1u) * RED_WORDS;
+            const bool decides = nijac > 0 && (nijac - 1) % 10 == 0;
+            const unsigned long long *prev = decides ? d.maxres + (((nijac - 1) / 10) & 1u) * RED_WORDS : nullptr;
+            ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
+            // setDarcyTopWallFixedFlow (bc_top == 1) writes dev_darcy_p, which
+            // the copy of p_new into p overwrites: it has no effect
+            // (device.cu:2284-2331)
+            // learned correction of the iterate this deciding sweep wrote
+            // (its kernels do nothing once the solve has ended); the sweep
+            // clears the correction's scale slot
+            const bool correct = decides && ctx->net && corrections < ctx->net_max_corr;
+            launch_darcy_sweep(s, da, d, buf[nijac & 1u], buf[(nijac & 1u) ^ 1u],
+                               check ? slot : nullptr, check ? next : nullptr, prev, h.tolerance,
+                               nijac - 1u, false, correct);
+            if (correct) {
+                const int nrc = darcy_correct(ctx, da, buf[(nijac & 1u) ^ 1u]);
+                if (nrc) return nrc;
+                ++corrections;
+            }
+        }
+        if (nijac == h.maxiter && (h.maxiter - 1) % 10 == 0)
+            launch_darcy_decide(s, d, d.maxres + (((h.maxiter - 1) / 10) & 1u) * RED_WORDS, h.tolerance,
+                                h.maxiter - 1);
+        HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
+        if (s == ctx->stream) {
+            const int rc = sync(ctx);
+            if (rc) return rc;
+        } else {
+            HIPCHK(hipStreamSynchronize(s));
+        }
+        want = (unsigned long long)nijac + 20u;
+    }
+    return SPH_OK;
+}
+
 // The sweeps of a solve as resident launches (resident.h): one launch up to
 // each learned correction (after sweeps 1, 11, 21, ...), then one to the end.
 // The launches alternate between the two iterate buffers; out is the one that
@@ -987,13 +1043,12 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
     const sph_state &h = ctx->hs.h;
     hipStream_t s = ctx->stream;
     const DarcyBuffers &d = ctx->dd;
-    const unsigned int chunk = 20000u;  // sweeps of a launch: some 30 ms
     std::vector<unsigned int> ends;
     int corrections = 0, cur = 0;
     std::memset(ctx->h_state, 0, 32);
     for (unsigned int it = 0; it < h.maxiter && ctx->h_state[0] == 0;) {
         const bool learned = ctx->net && corrections < ctx->net_max_corr;
-        const unsigned int len = learned ? (it == 0 ? 2u : 10u) : chunk;
+        const unsigned int len = learned ? (it == 0 ? 2u : 10u) : RES_CHUNK;
         const unsigned int end = it + std::min(len, h.maxiter - it);
         ResidentArgs a;
         bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->res_wait, a);
@@ -1035,6 +1090,50 @@ static int darcy_resident(sph_ctx *ctx, const DarcyArgs &da, double *const buf[2
     if (ctx->h_state[0] != 0)
         for (k = 0; ends[k] <= ctx->h_state[1];) ++k;
     out = ends.empty() ? 0 : (int)((k + 1) & 1u);
+    ctx->res.solves++;
+    return SPH_OK;
+}
+
+// The rest of a solve on stream s after its first `from` sweeps and its last
+// correction, in resident launches; the result is left where launches per sweep
+// leave it.  held: BarrierUses that the caller holds for s.  A launch that is
+// not to be, or whose wait runs out, leaves the sweeps from its first one on to
+// launches per sweep.
+static int darcy_resident_rest(sph_ctx *ctx, hipStream_t s, uint32_t held, const DarcyArgs &da, unsigned int from)
+{
+    const sph_state &h = ctx->hs.h;
+    const DarcyBuffers &d = ctx->dd;
+    double *const buf[2] = {d.p, d.p_new};
+    const size_t bytes = (size_t)dcells(h) * 8;
+    int cur = (int)(from & 1u);
+    std::memset(ctx->h_state, 0, 32);
+    for (unsigned int it = from; it < h.maxiter && ctx->h_state[0] == 0;) {
+        const unsigned int end = it + std::min(RES_CHUNK, h.maxiter - it);
+        ResidentArgs a;
+        const bool ok = resident_args(ctx->res, s, (int)da.nx, (int)da.ny, (int)da.nz, it, end, ctx->res_wait, a);
+        const bool ran = ok && launch_darcy_resident(s, ctx->device, ctx->res, a, da, d, buf[cur], buf[cur ^ 1],
+                                                     h.tolerance, held);
+        if (ran) {
+            HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            if (ctx->h_state[0] != RES_ABORT) {
+                cur ^= 1;
+                it = end;
+                continue;
+            }
+            resident_gave_up(ctx->res);
+            launch_fill_u32(s, (uint32_t *)(d.maxres + DARCY_STATE), 2, 0u);
+        } else if (ok) {
+            ctx->res.yielded++;
+        } else {
+            ctx->res.usable = false;
+        }
+        // a resident launch leaves the iterate it reads as it was
+        if (cur != (int)(it & 1u)) HIPCHK(hipMemcpyAsync(buf[it & 1u], buf[cur], bytes, hipMemcpyDeviceToDevice, s));
+        return darcy_launches(ctx, s, da, buf, it, ctx->net_max_corr);
+    }
+    const unsigned int ran = ctx->h_state[0] ? (unsigned int)ctx->h_state[1] + 1u : h.maxiter;
+    if (cur != (int)(ran & 1u)) HIPCHK(hipMemcpyAsync(buf[ran & 1u], buf[cur], bytes, hipMemcpyDeviceToDevice, s));
     ctx->res.solves++;
     return SPH_OK;
 }
@@ -1086,16 +1185,10 @@ static int darcy_step(sph_ctx *ctx, std::ofstream *convlog)
         launch_darcy_prepare(s, da, d);
         launch_fill_u32(s, (uint32_t *)d.maxres, 2 * DARCY_MAXRES_WORDS, 0u);
     }
-    // The sweeps (src/device.cu:2184-2386) ping-pong between the two
-    // buffers.  The convergence test of check sweep j (j % 10 == 0) runs on
-    // the device at the start of sweep j + 1, and once it ends the solve
-    // every later sweep returns at once.  The host enqueues sweeps in batches
-    // (the first as long as the last solve, each ending with a deciding
-    // sweep) and reads the solve state once per batch.
+    // The sweeps (src/device.cu:2184-2386)
     double *buf[2] = {d.p, d.p_new};
     int rc0 = net_ready(ctx);
     if (rc0) return rc0;
-    unsigned long long state = 0, last_nijac = 0, last_bits = 0;
     int out = 0;  // the buffer holding the solve's result
     int wrap = 0;
     bool resident = darcy_resident_form(da, wrap);
@@ -1105,54 +1198,12 @@ static int darcy_step(sph_ctx *ctx, std::ofstream *convlog)
     if (resident) {
         rc0 = darcy_resident(ctx, da, buf, resident, out);
         if (rc0) return rc0;
-        if (resident) {
-            state = ctx->h_state[0];
-            last_nijac = ctx->h_state[1];
-            last_bits = ctx->h_state[2];
-        }
     }
     if (!resident) {
-        int corrections = 0;
-        unsigned int nijac = 0;
-        unsigned long long want = std::max(12u, (ctx->jacobi_hint + 9u) / 10u * 10u + 2u);
-        while (nijac < h.maxiter && state == 0) {
-            const unsigned int end = (unsigned int)std::min<unsigned long long>(h.maxiter, want);
-            for (; nijac < end; ++nijac) {
-                const bool check = (nijac % 10 == 0);
-                // two check slots alternate: a check sweep zeroes the other one
-                unsigned long long *slot = d.maxres + ((nijac / 10) & 1u) * RED_WORDS;
-                unsigned long long *next = d.maxres + (((nijac / 10) & 1u) ^ 1u) * RED_WORDS;
-                const bool decides = nijac > 0 && (nijac - 1) % 10 == 0;
-                const unsigned long long *prev = decides ? d.maxres + (((nijac - 1) / 10) & 1u) * RED_WORDS : nullptr;
-                ProfScope ps(ctx, SPH_K_DARCY_SWEEP);
-                // setDarcyTopWallFixedFlow (bc_top == 1) writes dev_darcy_p, which
-                // the copy of p_new into p overwrites: it has no effect
-                // (device.cu:2284-2331)
-                // learned correction of the iterate this deciding sweep wrote
-                // (its kernels do nothing once the solve has ended); the sweep
-                // clears the correction's scale slot
-                const bool correct = decides && ctx->net && corrections < ctx->net_max_corr;
-                launch_darcy_sweep(s, da, d, buf[nijac & 1u], buf[(nijac & 1u) ^ 1u],
-                                   check ? slot : nullptr, check ? next : nullptr, prev, h.tolerance,
-                                   nijac - 1u, false, correct);
-                if (correct) {
-                    const int nrc = darcy_correct(ctx, da, buf[(nijac & 1u) ^ 1u]);
-                    if (nrc) return nrc;
-                    ++corrections;
-                }
-            }
-            if (nijac == h.maxiter && (h.maxiter - 1) % 10 == 0)
-                launch_darcy_decide(s, d, d.maxres + (((h.maxiter - 1) / 10) & 1u) * RED_WORDS, h.tolerance,
-                                    h.maxiter - 1);
-            HIPCHK(hipMemcpyAsync(ctx->h_state, d.maxres + DARCY_STATE, 32, hipMemcpyDeviceToHost, s));
-            int rc = sync(ctx);
-            if (rc) return rc;
-            state = ctx->h_state[0];
-            last_nijac = ctx->h_state[1];
-            last_bits = ctx->h_state[2];
-            want = (unsigned long long)nijac + 20u;
-        }
+        rc0 = darcy_launches(ctx, s, da, buf, 0u, 0);
+        if (rc0) return rc0;
     }
+    const unsigned long long state = ctx->h_state[0], last_nijac = ctx->h_state[1], last_bits = ctx->h_state[2];
     ctx->stats.corrections += ctx->h_state[3];
     // sweeps that ran: up to the deciding check, or all maxiter
     const unsigned int ran = state != 0 ? (unsigned int)last_nijac + 1u : h.maxiter;
@@ -2935,6 +2986,41 @@ static bool ens_fluid_current(const sph_ensemble *e)
 
 static MultiMap stage_map(const EnsStage &st) { return MultiMap{st.map, st.nbox}; }
 
+// The boxes still running go on in resident launches, one box after the other:
+// at most ENS_RESIDENT boxes, all of a form that allows it and past their
+// corrections.  A sweep of one launch for all costs 4.2 to 5.5 us however few
+// boxes run, a resident one 1.6 to 2.3 us per box, so that two boxes gain
+// and three do not.  64 boxes (406 sweeps in the median, 45,124 in one): 92 ms per
+// step, 233 with launches only, 131 box by box; 16 boxes of 400 to 425
+// sweeps: 6.9 either way, 14.7 box by box.  asked: the number of boxes of the last refusal.
+#define ENS_RESIDENT 2u
+static bool ens_take_resident(sph_ensemble *e, const std::vector<char> &running, int corrections,
+                              uint32_t &asked)
+{
+    uint32_t n = 0;
+    for (size_t i = 0; i < running.size(); ++i) {
+        if (!running[i]) continue;
+        if (++n > ENS_RESIDENT) return false;
+        if (ens_learned(e->boxes[e->fluid[i]]) && corrections < e->net_max_corr) return false;
+    }
+    if (n == asked) return false;
+    asked = n;
+    bool all = true;
+    for (size_t i = 0; i < running.size(); ++i) {
+        if (!running[i]) continue;
+        sph_ctx *c = e->boxes[e->fluid[i]];
+        const DarcyArgs da = darcy_args(c);
+        int wrap = 0;
+        if (!darcy_resident_form(da, wrap)) {
+            all = false;
+            continue;
+        }
+        if (!c->res.planned) resident_plan(c->res, c->device, (int)da.nx, (int)da.ny, (int)da.nz, wrap);
+        all = resident_ready(c->res) && all;
+    }
+    return all;
+}
+
 // One step of every fluid box (step_once with darcy_step, multi-box).
 static int ens_fluid_step(sph_ensemble *e)
 {
@@ -2980,7 +3066,8 @@ static int ens_fluid_step(sph_ensemble *e)
     // needed in its last solve (at least 12 sweeps in, then at least 20 more
     // per batch), and the next batch sweeps only the boxes whose solve had
     // not ended by then: a box with a long solve does not keep the others'
-    // blocks in every launch.  The sweeps an ended box skips would return
+    // blocks in every launch, and the last boxes' sweeps go on in resident
+    // launches (ens_take_resident).  The sweeps an ended box skips would return
     // at once, so the results are the same.
     const DarcyTask *tw = (const DarcyTask *)e->dm_sweep.tasks;
     const uint32_t maxiter = e->fl_maxiter;
@@ -3019,7 +3106,22 @@ static int ens_fluid_step(sph_ensemble *e)
     int corrections = 0;
     const DarcyTask *tn = (const DarcyTask *)e->dm_net.tasks;
     const MultiMap mn = stage_map(e->dm_net);
+    auto read_states = [&]() {
+        launch_dm_states(s, dt, nb, e->dm_states);
+        const hipError_t err = hipMemcpyAsync(e->dm_states_h, e->dm_states, 32 * nb, hipMemcpyDeviceToHost, s);
+        return err == hipSuccess ? hipStreamSynchronize(s) : err;
+    };
+    uint32_t asked = 0;
     while (nijac < maxiter && !all_ended) {
+        if (ens_take_resident(e, running, corrections, asked)) {
+            for (uint32_t i = 0; i < nb; ++i) {
+                if (!running[i]) continue;
+                sph_ctx *c = e->boxes[e->fluid[i]];
+                if ((rc = darcy_resident_rest(c, s, 1u, darcy_args(c), nijac))) return ens_fail(e, rc, c->err);
+            }
+            HIPCHK_E(read_states());
+            break;
+        }
         const unsigned int end = (unsigned int)std::min<unsigned long long>(maxiter, want);
         for (; nijac < end; ++nijac) {
             const bool decides = nijac > 0 && (nijac - 1) % 10 == 0;
@@ -3034,9 +3136,7 @@ static int ens_fluid_step(sph_ensemble *e)
             }
         }
         if (nijac == maxiter && (maxiter - 1) % 10 == 0) launch_dm_decide(s, dt, nb, maxiter - 1);
-        launch_dm_states(s, dt, nb, e->dm_states);
-        HIPCHK_E(hipMemcpyAsync(e->dm_states_h, e->dm_states, 32 * nb, hipMemcpyDeviceToHost, s));
-        HIPCHK_E(hipStreamSynchronize(s));
+        HIPCHK_E(read_states());
         all_ended = true;
         bool changed = false;
         for (uint32_t i = 0; i < nb; ++i) {
@@ -3044,6 +3144,9 @@ static int ens_fluid_step(sph_ensemble *e)
             changed = changed || (run != (running[i] != 0));
             running[i] = run ? 1 : 0;
             all_ended = all_ended && !run;
+            // past its last solve's sweeps: looked at again 20 sweeps or an
+            // eighth later, not at the end of the longest box's solve
+            if (target[i] <= nijac) target[i] = nijac + std::max(20u, nijac / 80u * 10u);
         }
         if (changed && !all_ended) HIPCHK_E(remap());
         want = next_end((unsigned long long)nijac + 20u);

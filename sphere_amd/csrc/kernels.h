@@ -354,7 +354,7 @@ bool darcy_resident_form(const DarcyArgs &d, int &wrap);
 // (false: not now, resident_begin)
 bool launch_darcy_resident(hipStream_t s, int device, const Resident &r, const ResidentArgs &a,
                            const DarcyArgs &d, const DarcyBuffers &b, const double *p_in, double *p_out,
-                           double tolerance);
+                           double tolerance, uint32_t held = 0u);
 void launch_darcy_residual_max(hipStream_t s, const DarcyArgs &d, const DarcyBuffers &b, const double *p,
                                bool free_running);
 // the network input of iterate p: FP32 rows of 3 (input) and/or the

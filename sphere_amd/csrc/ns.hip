@@ -894,7 +894,7 @@ int ns_resident(sph_ns *n, bool &resident, bool &converged, unsigned &nijac)
 {
     const sph_ns_params &P = n->P;
     const NsGrid &g = n->g;
-    const unsigned chunk = 20000u;  // iterations of a launch: some 30 ms
+    const unsigned chunk = RES_CHUNK;
     const bool keep = P.maxiter > chunk;
     if (keep && !n->eps_start &&
         hipMalloc((void **)&n->eps_start, n->nc * sizeof(double)) != hipSuccess) {

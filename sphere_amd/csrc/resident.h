@@ -49,6 +49,7 @@
 #define RES_SPIN (1u << 20)   // default bound of a wait in polls (about 1 s)
 #define RES_CELL_THREADS 960  // threads owning cells: a block's 1024 less the gathering wave
 #define RES_CHECK 10u         // iterations between residual tests
+#define RES_CHUNK 20000u      // iterations of a launch at most: some 30 ms
 #define RES_LAG 3u            // iterations between a test and its verdict
 // The wait before a wave reads its halo, in units of 4 cycles: longer by
 // RES_MORE after an iteration in which a value came late, else shorter by
@@ -108,8 +109,9 @@ void resident_gave_up(Resident &r);
 bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t it0, uint32_t it1,
                    const ResidentWait &wait, ResidentArgs &out);
 // Resident launches of one device wait for each other: call before and after
-// the launch.  False, and then no launch: a BarrierUse of the device is held.
-bool resident_begin(int device, hipStream_t s);
+// the launch.  False, and then no launch: a BarrierUse of the device is held,
+// beside `held` that the caller itself holds for stream s.
+bool resident_begin(int device, hipStream_t s, uint32_t held);
 void resident_end(int device, hipStream_t s);
 
 // Held while stream s of a device may run grid barriers.
@@ -463,9 +465,10 @@ __global__ void __launch_bounds__(1024) k_resident_jacobi(ResidentArgs r, Op op)
 
 // false: not now (resident_begin)
 template <class Op>
-bool resident_launch(const Resident &r, int device, hipStream_t s, const ResidentArgs &a, const Op &op)
+bool resident_launch(const Resident &r, int device, hipStream_t s, const ResidentArgs &a, const Op &op,
+                     uint32_t held = 0u)
 {
-    if (!resident_begin(device, s)) return false;
+    if (!resident_begin(device, s, held)) return false;
     if (r.per_thread == 1)
         hipLaunchKernelGGL((k_resident_jacobi<Op, 1>), dim3(r.tiles), dim3(r.threads), r.lds, s, a, op);
     else

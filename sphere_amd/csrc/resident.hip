@@ -124,11 +124,11 @@ bool resident_args(Resident &r, hipStream_t s, int nx, int ny, int nz, uint32_t 
     return true;
 }
 
-bool resident_begin(int device, hipStream_t s)
+bool resident_begin(int device, hipStream_t s, uint32_t held)
 {
     DeviceOrder &o = g_order[device];
     o.m.lock();
-    if (o.barriers) {
+    if (o.barriers > held) {
         o.m.unlock();
         return false;
     }
