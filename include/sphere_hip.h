@@ -188,9 +188,9 @@ int sph_set_contact_slots(sph_ctx *ctx, int nc);
  * does a grid that leaves no room for it); cap is the number of list entries
  * per particle (1..128, default 128; a particle with more neighbours than
  * that is searched over the cells, and the lists are then rebuilt every
- * step).  Takes effect at the next load.  In list mode the cell sort runs
- * only on rebuild steps, so sph_read_sort returns the arrays of the last
- * rebuild. */
+ * step).  Takes effect at the next load.  In list mode without a fluid the
+ * cell sort runs only on rebuild steps, so sph_read_sort returns the arrays of
+ * the last rebuild. */
 int sph_set_neighbor_lists(sph_ctx *ctx, double skin_fraction, int cap);
 int sph_get_neighbor_stats(sph_ctx *ctx, sph_neighbor_stats *out);
 
@@ -199,7 +199,8 @@ int sph_get_neighbor_stats(sph_ctx *ctx, sph_neighbor_stats *out);
  * barriers, followed by the list build; both are launched every step and
  * return at once unless the rebuild flag is set.  fused = 0: the sort
  * passes, reorder and list build are separate launches that each return at
- * once between rebuilds.  Runs with fluid rebuild every step and always use
+ * once between rebuilds.  Runs with a fluid, which reads the sorted arrays,
+ * sort and reorder every step, build lists on flagged steps, and always use
  * the separate launches.  Both give the same arrays.  Takes effect at the
  * next load. */
 int sph_set_rebuild_kernel(sph_ctx *ctx, int fused);

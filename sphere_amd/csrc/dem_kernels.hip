@@ -12,7 +12,8 @@
 //   k_bond_gather     and a per-particle gather in ascending bond order
 //   k_integrate       integrate (src/integration.cuh:14-305) fused with the
 //                     256-wide block reduction of summation (:309-341)
-//   k_integrate_walls integrateWalls (src/integration.cuh:344-450)
+//   k_step_end        integrateWalls (src/integration.cuh:344-450) and the
+//                     clock's advance, mostly inside the next k_topology_lists
 #include "kernels.h"
 
 // ------------------------------------------------------------------
@@ -633,8 +634,8 @@ void launch_nl_build(hipStream_t s, const StepArgs &a, const NLArgs &n, const De
 // list path the radix passes, the cell clear and the reorder run as one
 // kernel whose phases are separated by grid barriers, and the list build
 // follows as one more launch (in small boxes it joins the kernel); a step
-// without a rebuild then costs two dispatches, or one, instead of nine.  The grid is at most one block per compute
-// unit, so every block is resident.
+// without a rebuild then costs two dispatches, or one, instead of nine.  The
+// grid is at most one block per compute unit, so every block is resident.
 
 // Grid barrier.  bar[0] counts arrivals, bar[1] is the generation; `gen` is
 // the generation this block waits to see end.  A waiter that spins longer

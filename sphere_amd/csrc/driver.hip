@@ -134,7 +134,7 @@ static int fail(sph_ctx *ctx, int code, const std::string &msg)
 // profiling with HIP events on the context stream
 // ------------------------------------------------------------------
 
-static size_t prof_event(sph_ctx *ctx, hipStream_t s)
+static size_t prof_event(sph_ctx *ctx)
 {
     if (ctx->ev_used == ctx->ev_pool.size()) {
         hipEvent_t e;
@@ -142,24 +142,22 @@ static size_t prof_event(sph_ctx *ctx, hipStream_t s)
         ctx->ev_pool.push_back(e);
     }
     size_t i = ctx->ev_used++;
-    (void)hipEventRecord(ctx->ev_pool[i], s);
+    (void)hipEventRecord(ctx->ev_pool[i], ctx->stream);
     return i;
 }
 
 struct ProfScope {
     sph_ctx *ctx;
     int k;
-    hipStream_t s;
     size_t e0;
-    ProfScope(sph_ctx *c, int kid, hipStream_t st = nullptr)
-        : ctx(c), k(kid), s(st ? st : c->stream), e0((size_t)-1)
+    ProfScope(sph_ctx *c, int kid) : ctx(c), k(kid), e0((size_t)-1)
     {
-        if (ctx->prof) e0 = prof_event(ctx, s);
+        if (ctx->prof) e0 = prof_event(ctx);
     }
     ~ProfScope()
     {
         if (ctx->prof && e0 != (size_t)-1) {
-            size_t e1 = prof_event(ctx, s);
+            size_t e1 = prof_event(ctx);
             if (e1 != (size_t)-1) ctx->ev_pending.emplace_back(k, e0, e1);
         }
     }

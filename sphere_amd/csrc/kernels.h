@@ -275,11 +275,11 @@ StepEnd step_end(const StepArgs &a, const DemBuffers &b);
 HashTask hash_task(const StepArgs &a, const NLArgs &n, const DemBuffers &b, uint32_t cur,
                    uint32_t force);
 BondGatherTask bond_gather_task(const DemBuffers &b);
-// Blocks a box needs in each multi-box stage.
-// grains of one wave in the search and contact kernels, for a launch over np
-// grains, and the waves that np grains then take
+// Grains of one wave in the search and contact kernels, for a launch over np
+// grains, and the waves (blocks) that np grains then take.
 uint32_t grains_per_wave(uint64_t np);
 uint32_t wave_blocks(uint32_t np, uint32_t gpw);
+// Blocks of the list build.
 uint32_t nl_build_blocks(uint32_t np);
 // Multi-box launches of `blocks` blocks (the last start plus its count,
 // rounded up) over device task arrays; near/hertz pick the kernel variant
@@ -294,8 +294,7 @@ void launch_bonds_multi(hipStream_t s, const BondTask *t, MultiMap m, uint32_t b
 void launch_integrate_multi(hipStream_t s, const IntegrateTask *t, MultiMap m, uint32_t blocks);
 void launch_hash_multi(hipStream_t s, const HashTask *t, MultiMap m, uint32_t blocks);
 void launch_bond_gather_multi(hipStream_t s, const BondGatherTask *t, MultiMap m, uint32_t blocks);
-// one block per task
-// the end of a step of n boxes: walls and clock
+// The end of a step of n boxes, walls and clock: one block per task.
 void launch_step_end_multi(hipStream_t s, const StepEndTask *t, uint32_t n);
 
 // A max over all the blocks of a launch (the bit pattern of a non-negative
