@@ -647,20 +647,20 @@ public:
     {
         std::lock_guard<std::mutex> lock(m_);
         if (--contexts_ == 0)
-            while (!idle_.empty()) drop(idle_.size() - 1);
+            while (n_) drop(n_ - 1u);
     }
     // the smallest piece that holds `bytes`, else a new one of the next power of
     // two; p is null where none can be made
     Pinned take(size_t bytes)
     {
         std::lock_guard<std::mutex> lock(m_);
-        size_t best = idle_.size();
-        for (size_t k = 0; k < idle_.size(); ++k)
-            if (idle_[k].bytes >= bytes && (best == idle_.size() || idle_[k].bytes < idle_[best].bytes)) best = k;
+        uint32_t best = n_;
+        for (uint32_t k = 0; k < n_; ++k)
+            if (idle_[k].bytes >= bytes && (best == n_ || idle_[k].bytes < idle_[best].bytes)) best = k;
         Pinned q;
-        if (best < idle_.size()) {
+        if (best < n_) {
             q = idle_[best];
-            idle_.erase(idle_.begin() + (long)best);
+            idle_[best] = idle_[--n_];
             return q;
         }
         for (q.bytes = size_t(256) << 10; q.bytes < bytes;) q.bytes *= 2;
@@ -673,22 +673,23 @@ public:
     void give(const Pinned &q)
     {
         std::lock_guard<std::mutex> lock(m_);
-        idle_.push_back(q);
-        if (idle_.size() <= PINNED_IDLE) return;
-        size_t least = 0;
-        for (size_t k = 1; k < idle_.size(); ++k)
+        idle_[n_++] = q;
+        if (n_ <= PINNED_IDLE) return;
+        uint32_t least = 0;
+        for (uint32_t k = 1; k < n_; ++k)
             if (idle_[k].bytes < idle_[least].bytes) least = k;
         drop(least);
     }
 
 private:
-    void drop(size_t k)
+    void drop(uint32_t k)
     {
         (void)hipHostFree(idle_[k].p);
-        idle_.erase(idle_.begin() + (long)k);
+        idle_[k] = idle_[--n_];
     }
     std::mutex m_;
-    std::vector<Pinned> idle_;
+    Pinned idle_[PINNED_IDLE + 1u];
+    uint32_t n_ = 0;
     size_t contexts_ = 0;
 };
 static PinnedPool g_pinned;
