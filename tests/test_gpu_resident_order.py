@@ -40,7 +40,7 @@ def _afloat():
 def test_solve_beside_another_threads_rebuilds():
     ref, e = _engine(_fluid()), _engine(_fluid())
     grains, started = _engine(_afloat()), threading.Event()
-    steps = 20000
+    steps = 40000
     alone = _engine(_afloat())
     alone.step(steps)
 
